@@ -9,6 +9,10 @@
 // whose RK23 pass reads the cluster descriptor from a copy in LDS, used when
 // every instance of the launch is RK23 (ofx_backend_rkl.hip).
 enum { XMODE_RK23_LDS = 2 };
+// Bits 4..6: the wave kernel (ofx_wave_impl.h) with this many points a thread
+// (1, 2 or 4); bit 7: its form for workgroups of more than 256 threads.  The
+// other bits are then 0.
+enum { XMODE_WAVE_SHIFT = 4, XMODE_WAVE_MASK = 0x70, XMODE_WAVE_WIDE = 0x80 };
 
 namespace ofx {
 

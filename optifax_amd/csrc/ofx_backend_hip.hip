@@ -26,10 +26,15 @@ __global__ void __launch_bounds__(512) pass_kernel(LaunchArgs a) {
 
 // the RK23 variant's kernels (ofx_backend_rkl.hip)
 const void* rkl_kernel(int precision, int xmode);
+// the wave kernels (ofx_backend_wave.hip)
+const void* wave_kernel_fn(int precision, int points, bool wide);
 
 // the kernel instantiation for a precision and xmode (exchange mode in bit 0,
-// XMODE_RK23_LDS in bit 1)
+// XMODE_RK23_LDS in bit 1, the wave kernel's points a thread in bits 4..6)
 static const void* pass_fn(int precision, int xmode) {
+  if (xmode & XMODE_WAVE_MASK)
+    return wave_kernel_fn(precision, (xmode & XMODE_WAVE_MASK) >> XMODE_WAVE_SHIFT,
+                          (xmode & XMODE_WAVE_WIDE) != 0);
   if (xmode & XMODE_RK23_LDS) return rkl_kernel(precision, xmode & 1);
   xmode &= 1;
   if (precision == OFX_F64)
@@ -143,7 +148,10 @@ int be_create(int device, Backend** out, DeviceInfo* info) {
     const int dyn = info->lds_max - 1024;
     bool ok = true;
     for (int prec : {OFX_F32, OFX_F64})
-      for (int xm : {XM_TAGS, XM_BARRIER, XM_TAGS | XMODE_RK23_LDS, XM_BARRIER | XMODE_RK23_LDS})
+      for (int xm : {XM_TAGS, XM_BARRIER, XM_TAGS | XMODE_RK23_LDS, XM_BARRIER | XMODE_RK23_LDS,
+                     1 << XMODE_WAVE_SHIFT, 2 << XMODE_WAVE_SHIFT, 4 << XMODE_WAVE_SHIFT,
+                     1 << XMODE_WAVE_SHIFT | XMODE_WAVE_WIDE, 2 << XMODE_WAVE_SHIFT | XMODE_WAVE_WIDE,
+                     4 << XMODE_WAVE_SHIFT | XMODE_WAVE_WIDE})
         ok = ok && hipFuncSetAttribute(pass_fn(prec, xm), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        dyn) == hipSuccess;
     if (!ok)

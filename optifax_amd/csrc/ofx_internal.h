@@ -93,6 +93,7 @@ struct LaunchArgs {
   const int* wg_rank;      // per workgroup: rank within its cluster
   const void* twiddle;     // NMAX complex: exp(-2 pi i m / NMAX)
   int nmax;                // twiddle table size (largest N in the launch)
+  int block;               // threads per workgroup
   int trips;               // 0: single pass (MEX mode); >0: round trips
   double conv_tol;         // stop an instance when conv metric < tol (<=0 never)
   unsigned long long timeout_ticks;  // barrier spin limit in wall-clock ticks

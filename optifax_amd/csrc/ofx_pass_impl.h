@@ -1619,21 +1619,14 @@ OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const Inst
   }
 }
 
-// (with OFX_RKL, cdl: workgroup-shared storage for the descriptor's copy)
-template <typename R, int XM>
-OFX_DEV void cluster_main(const LaunchArgs& a, int wg, cpx<R>* lds, double* red,
-                          int* sflag OFX_CDL_PARAM) {
-  const int ci = a.wg_cluster[wg];
-  if (ci < 0) return;
-  const ClusterDesc& cd = a.clusters[ci];
-#ifdef OFX_RKL
-  if (OFX_TID == 0) *cdl = cd;
-  OFX_SYNC();
-  const ClusterDesc& cdr = *cdl;
-#endif
-  const int rank = a.wg_rank[wg];
-  SyncState sy;
+// A member's exchange state at the start of a launch, and its placement
+// record (hardware XCC id).
+OFX_DEV void member_begin(const LaunchArgs& a, const ClusterDesc& cd, int wg, int rank, int* sflag,
+                          SyncState& sy) {
 #ifdef OFX_EMU
+  (void)a;
+  (void)wg;
+  (void)rank;
   sy.base = __atomic_load_n(cd.epoch, __ATOMIC_RELAXED);
 #else
   sy.base = __hip_atomic_load(cd.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1649,13 +1642,11 @@ OFX_DEV void cluster_main(const LaunchArgs& a, int wg, cpx<R>* lds, double* red,
     if (a.xcc_ids) a.xcc_ids[wg] = x;
   }
 #endif
-  for (int ii = 0; ii < cd.n_inst; ii++) {
-    const int id = a.inst_order[cd.first_inst + ii];
-    run_instance<R, XM>(a, cd, a.inst[id], rank, lds, red, sflag, sy OFX_RKL_ARG);
-    if (flag_load(cd.abort_flag)) break;
-  }
-  // the tags this member used end at base + nx: the next launch starts past
-  // the largest over the cluster
+}
+
+// the tags this member used end at base + nx: the next launch starts past
+// the largest over the cluster
+OFX_DEV void member_end(const ClusterDesc& cd, const SyncState& sy) {
   if (OFX_TID == 0) {
 #ifdef OFX_EMU
     unsigned cur = __atomic_load_n(cd.epoch + 1, __ATOMIC_RELAXED);
@@ -1667,6 +1658,29 @@ OFX_DEV void cluster_main(const LaunchArgs& a, int wg, cpx<R>* lds, double* red,
     __hip_atomic_fetch_max(cd.epoch + 1, sy.nx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #endif
   }
+}
+
+// (with OFX_RKL, cdl: workgroup-shared storage for the descriptor's copy)
+template <typename R, int XM>
+OFX_DEV void cluster_main(const LaunchArgs& a, int wg, cpx<R>* lds, double* red,
+                          int* sflag OFX_CDL_PARAM) {
+  const int ci = a.wg_cluster[wg];
+  if (ci < 0) return;
+  const ClusterDesc& cd = a.clusters[ci];
+#ifdef OFX_RKL
+  if (OFX_TID == 0) *cdl = cd;
+  OFX_SYNC();
+  const ClusterDesc& cdr = *cdl;
+#endif
+  const int rank = a.wg_rank[wg];
+  SyncState sy;
+  member_begin(a, cd, wg, rank, sflag, sy);
+  for (int ii = 0; ii < cd.n_inst; ii++) {
+    const int id = a.inst_order[cd.first_inst + ii];
+    run_instance<R, XM>(a, cd, a.inst[id], rank, lds, red, sflag, sy OFX_RKL_ARG);
+    if (flag_load(cd.abort_flag)) break;
+  }
+  member_end(cd, sy);
 }
 
 }  // namespace ofx

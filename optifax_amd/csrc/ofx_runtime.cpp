@@ -129,6 +129,48 @@ size_t lds_bytes_for(int n1, int n2, int C, int method, size_t csz) {
           ((size_t)W * (size_t)n2 + 1) / 2) * csz + 16 + (size_t)(n1 + n2) * 16;
 }
 
+// LDS of a workgroup of the wave kernel: A0 with its halo, the column slots
+// (272 elements each 256) and the row slots (ofx_wave_impl.h)
+size_t wave_lds_bytes(int n1, int n2, int C, size_t csz) {
+  const size_t W = n1 / C, Rr = n2 / C, LC = W + 4;
+  return (LC * (size_t)(n2 + 1) +
+          ((LC * n2 + 255) / 256 + (Rr * n1 + 255) / 256) * 272) * csz;
+}
+
+// Points a thread with which the wave kernel can run an instance (1, 2 or 4),
+// or 0 when it cannot: Heun, transforms of at most 256, at most 4 points a
+// thread, every column row with a thread, at most two error records a lane.
+int wave_points(const ofx_pass_params& p, int n1, int C, int block, size_t csz, int lds_max) {
+  const int n2 = p.n / n1, share = p.n / C;
+  if (p.method != OFX_METHOD_HEUN || n1 > 256 || n2 > 256 || C > 128 || ilog2i(block) < 0 ||
+      block < n2 || share > 4 * block || (int)wave_lds_bytes(n1, n2, C, csz) > lds_max - 1024)
+    return 0;
+  return share > 2 * block ? 4 : share > block ? 2 : 1;
+}
+
+// Workgroups per instance for the wave kernel, or 0 when it does not apply.
+// A grid of up to 2^10 points runs in one workgroup without any exchange; a
+// larger one takes the workgroups that measured fastest (us per adaptive
+// step, FP32 / FP64, one instance; the general kernel at its best geometry
+// after the colon):
+//   2^9   1 workgroup 5.5 / 6.1, 8: 6.8 / 7.6            : 7.9 / 8.9
+//   2^10  1: 6.5 / 7.9, 16: 7.5 / 8.1                    : 8.7 / -
+//   2^11  1: 8.4 / 15.8, 16: 7.5 / 8.6, 32: 7.3 / 8.2    : 9.0 / 10.6
+//   2^12  16: 8.3 / 10.2, 32: 8.1 / 10.5                 : 10.2 / 11.7
+//   2^13  16: 9.4 / 11.9, 32: 9.1 / 11.8                 : 11.0 / 12.8
+//   2^14  32: 10.6 / 14.8, 64: 9.2 / 11.8, 128: 9.9 / 12.6 : 12.2 / 14.5
+//   2^15  64: 10.0 / 12.9, 128: 10.0 / 13.7              : 12.7 / 16.1
+//   2^16  64: 12.4 / 18.6, 128: 12.0 / 17.7              : 15.4 / -
+// With several instances each takes what keeps them all resident, down to 4
+// points a thread of 256 (2^14 at 16 workgroups: 11.3 against 16.5).
+int wave_cluster(const ofx_pass_params& p, int n1, int n_inst, int cus) {
+  const int n = p.n;
+  if (p.method != OFX_METHOD_HEUN || n1 > 256 || n / n1 > 256) return 0;
+  int C = n <= 1024 ? 1 : n <= 8192 ? 32 : n <= 16384 ? 64 : 128;
+  while (C > 1 && (long long)n_inst * C > cus) C >>= 1;
+  return n / C <= 1024 && (long long)n_inst * C <= cus ? C : 0;
+}
+
 // largest cluster size the method allows (RK23 exchanges 3 boundary columns
 // of K4 with each neighbour, so each workgroup owns at least 4 columns)
 int max_cluster(int method, int n1, int n2) {
@@ -269,12 +311,14 @@ int plan_instance(ofx_context* ctx, const ofx_pass_params& p, int n_inst, const 
     if (ilog2i(C) < 0 || C > cmax ||
         (int)lds_bytes_for(n1, n2, C, meth, csz) > ctx->info.lds_max - 1024)
       return fail(ctx, OFX_E_ARG, "cluster size %d is invalid for N=%d (n1=%d)", C, n, n1);
+  } else if (const int Cw = tune && tune->exchange == 2 ? 0
+                            : wave_cluster(p, n1, n_inst, ctx->info.cus)) {
+    C = Cw;
   } else {
-    // Spread a small batch over more workgroups: a step's latency is set by
-    // the per-workgroup share until it falls to ~256 points (measured on
-    // N = 2^15, FP32 / FP64 us per adaptive step: 20.1 / 24.2 at 32
-    // workgroups, 16.6 / 21.1 at 64, 15.5 / 19.6 at 128 with 256-thread
-    // workgroups).
+    // The general kernel: spread a small batch over more workgroups until a
+    // share falls to ~256 points (measured on N = 2^15, FP32 / FP64 us per
+    // adaptive step: 20.1 / 24.2 at 32 workgroups, 16.6 / 21.1 at 64, 15.5 /
+    // 19.6 at 128 with 256-thread workgroups).
     const int slots_est = ctx->info.cus;
     while (C * 2 <= cmax && (long long)n_inst * C * 2 <= slots_est && C * 2 <= 128 &&
            n / (C * 2) >= 256)
@@ -285,13 +329,30 @@ int plan_instance(ofx_context* ctx, const ofx_pass_params& p, int n_inst, const 
   return OFX_OK;
 }
 
-// Threads per workgroup: 256 once every cluster has 128 members or more (a
-// share of <= 256 points per workgroup), 512 below.
-int plan_block(ofx_context* ctx, const ofx_tuning* tune, int cmin, int* block) {
+// Threads per workgroup of the wave kernel for one instance: a wave for each
+// 256 elements of the own and halo columns (the step's longest transform
+// phase), 256 in a cluster of one for the stages' sake; at most 512 with FP32
+// fields (N = 2^16 at 128 workgroups: 12.0 us per step with 512 threads, 13.2
+// with 256) and 256 with FP64 fields (whose 512-thread form spills: 36 against
+// 17.7).  0 when the wave kernel cannot run the instance.
+int wave_block(const ofx_pass_params& p, int n1, int C, size_t csz, int lds_max) {
+  const int n2 = p.n / n1, el = C == 1 ? p.n : (n1 / C + 4) * n2;
+  int block = 64;
+  while (block < el / 4 || block < n2 || (C == 1 && block < std::min(p.n, 256))) block <<= 1;
+  block = std::min(block, csz == 8 ? 512 : 256);
+  return wave_points(p, n1, C, block, csz, lds_max) ? block : 0;
+}
+
+// Threads per workgroup: the wave kernel's when it can run every instance
+// (wblock), else 256 once every cluster has 128 members or more (a share of
+// <= 256 points per workgroup), 512 below.
+int plan_block(ofx_context* ctx, const ofx_tuning* tune, int cmin, int wblock, int* block) {
   const int exchange = tune ? tune->exchange : 0;
   if (exchange < 0 || exchange > 2)
     return fail(ctx, OFX_E_ARG, "exchange=%d must be 0 (auto), 1 (tags) or 2 (barrier)", exchange);
-  *block = (tune && tune->block) ? tune->block : (cmin >= 128 ? 256 : 512);
+  *block = (tune && tune->block)        ? tune->block
+           : wblock && exchange != 2 ? wblock
+                                     : (cmin >= 128 ? 256 : 512);
   if (*block < 64 || *block > 512 || (*block & 63))
     return fail(ctx, OFX_E_ARG, "block=%d must be a multiple of 64 in [64,512]", *block);
   return OFX_OK;
@@ -393,10 +454,14 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
     }
   }
   r->nmax = nmax;
-  int cmin0 = 1 << 30;
-  for (int i = 0; i < n_inst; i++) cmin0 = std::min(cmin0, r->inst_C[i]);
+  int cmin0 = 1 << 30, wblock = 0;
+  for (int i = 0; i < n_inst; i++) {
+    cmin0 = std::min(cmin0, r->inst_C[i]);
+    const int b = wave_block(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->csz, ctx->info.lds_max);
+    wblock = i && !wblock ? 0 : b ? std::max(wblock, b) : 0;
+  }
   const int exchange = tune ? tune->exchange : 0;
-  st = plan_block(ctx, tune, cmin0, &r->block);
+  st = plan_block(ctx, tune, cmin0, wblock, &r->block);
   if (st) {
     delete r;
     return st;
@@ -408,8 +473,23 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
     lds = std::max(lds, lds_bytes_for(n1, n2, r->inst_C[i], specs[i].pass.method, r->csz));
     cmin = std::min(cmin, r->inst_C[i]);
   }
-  r->lds = lds;
   r->xmode = exchange_mode(exchange, cmin);
+  // the wave kernel when it can run every instance
+  int points = 0;
+  for (int i = 0; i < n_inst && exchange != 2; i++) {
+    const int w = wave_points(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->block, r->csz,
+                              ctx->info.lds_max);
+    points = w ? std::max(points, w) : 0;
+    if (!w) break;
+  }
+  if (points) {
+    r->xmode = (points << XMODE_WAVE_SHIFT) | (r->block > 256 ? XMODE_WAVE_WIDE : 0);
+    lds = 0;
+    for (int i = 0; i < n_inst; i++)
+      lds = std::max(lds, wave_lds_bytes(r->inst_n1[i], specs[i].pass.n / r->inst_n1[i],
+                                         r->inst_C[i], r->csz));
+  }
+  r->lds = lds;
   bool all_rk23 = n_inst > 0;
   for (int i = 0; i < n_inst; i++) all_rk23 = all_rk23 && specs[i].pass.method == OFX_METHOD_RK23;
   if (all_rk23) r->xmode |= XMODE_RK23_LDS;
@@ -680,6 +760,7 @@ static LaunchArgs make_args(ofx_opo* r, int trips, double tol) {
   a.wg_rank = r->wgr_d;
   a.twiddle = r->twiddle;
   a.nmax = r->nmax;
+  a.block = r->block;
   a.trips = trips;
   a.conv_tol = tol;
   // exchange wait limit in wall-clock ticks
@@ -1157,11 +1238,14 @@ extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params*
   // cluster per instance, all resident at once)
   int C = 0, n1 = 0, block = 0;
   st = plan_instance(ctx, *p, batch, nullptr, 0, 0, 8, &C, &n1);
-  if (!st) st = plan_block(ctx, nullptr, C, &block);
+  if (!st)
+    st = plan_block(ctx, nullptr, C, wave_block(*p, n1, C, 8, ctx->info.lds_max), &block);
   if (st) return st;
   const int n2 = n / n1;
-  const int xmode = exchange_mode(0, C);
-  const size_t lds = lds_bytes_for(n1, n2, C, method, 8);
+  const int points = wave_points(*p, n1, C, block, 8, ctx->info.lds_max);
+  const int xmode = points ? (points << XMODE_WAVE_SHIFT) | (block > 256 ? XMODE_WAVE_WIDE : 0)
+                           : exchange_mode(0, C);
+  const size_t lds = points ? wave_lds_bytes(n1, n2, C, 8) : lds_bytes_for(n1, n2, C, method, 8);
   const int bpc = be_blocks_per_cu(ctx->be, OFX_F32, xmode, block, lds);
   if (bpc < 1)
     return fail(ctx, OFX_E_ARG, "kernel cannot launch with block=%d and %zu bytes of LDS", block, lds);
@@ -1317,6 +1401,7 @@ extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params*
   a.wg_rank = (const int*)(S + o_wgr);
   a.twiddle = S + o_tw;
   a.nmax = n;
+  a.block = block;
   a.trips = 0;
   a.conv_tol = 0.0;
   a.timeout_ticks = (unsigned long long)((double)ctx->info.wallclock_khz * 1000.0 * 10.0);

@@ -21,6 +21,7 @@
 #include "../../include/optifax_hip.h"
 #include "../../optifax_amd/csrc/ofx_backend.h"
 #include "../../optifax_amd/csrc/ofx_pass_impl.h"
+#include "../../optifax_amd/csrc/ofx_wave_impl.h"
 
 namespace ofx {
 
@@ -90,11 +91,25 @@ static void run_wg(const LaunchArgs* a, int wg, size_t lds) {
   cluster_main<R, XM>(*a, wg, reinterpret_cast<cpx<R>*>(mem.data()), red, sflag);
 }
 
+// the wave kernel: a workgroup's threads are walked phase by phase
+template <typename R, int S>
+static void run_wave(const LaunchArgs* a, int wg, size_t lds) {
+  std::vector<unsigned char> mem(lds + 64);
+  std::vector<WvThread<R, S>> thr((size_t)a->block);
+  double red[64];
+  int sflag[4];
+  wave_main<R, S>(*a, wg, reinterpret_cast<cpx<R>*>(mem.data()), red, sflag, thr.data());
+}
+template <typename R>
+static void (*wave_fn(int points))(const LaunchArgs*, int, size_t) {
+  return points == 4 ? run_wave<R, 4> : points == 2 ? run_wave<R, 2> : run_wave<R, 1>;
+}
+
 int be_launch(Backend* b, const LaunchArgs& a, int precision, int xmode, int grid, int block,
               size_t lds, unsigned* const* zp, const size_t* zw, int nz, unsigned* ep, int nep,
               const void* key, int replays) {
-  (void)block;
   (void)key;
+  (void)block;
   const int reps = replays > 0 ? replays : 1;
   for (int rep = 0; rep < reps; rep++) {
     for (int i = 0; i < nz; i++) memset(zp[i], 0, zw[i] * sizeof(unsigned));
@@ -105,7 +120,10 @@ int be_launch(Backend* b, const LaunchArgs& a, int precision, int xmode, int gri
     std::vector<std::thread> th;
     const bool bar = (xmode & 1) == XM_BARRIER;
     for (int wg = 0; wg < grid; wg++) {
-      if (xmode & XMODE_RK23_LDS)
+      if (xmode & XMODE_WAVE_MASK) {
+        const int pts = (xmode & XMODE_WAVE_MASK) >> XMODE_WAVE_SHIFT;
+        th.emplace_back(precision == OFX_F64 ? wave_fn<double>(pts) : wave_fn<float>(pts), &a, wg, lds);
+      } else if (xmode & XMODE_RK23_LDS)
         th.emplace_back(emu_rkl_fn(precision, xmode & 1), &a, wg, lds);
       else if (precision == OFX_F64)
         th.emplace_back(bar ? run_wg<double, XM_BARRIER> : run_wg<double, XM_TAGS>, &a, wg, lds);
