@@ -3,7 +3,7 @@
 // Stockham FFTs and up to 0.42 n twiddles: n <= 2^13 in FP32, 2^12 in FP64
 // within the 160 KB of LDS),
 // Dormand-Prince 5(4) with ode45's step control, outputs at the requested
-// points.  The body is ofx_gnlse_impl.h.
+// points.  The body is ofx_gnlse_impl.h, for long grids ofx_gnlse_wide.h.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <string.h>
@@ -13,6 +13,7 @@
 
 #include "../../include/optifax_hip.h"
 #include "ofx_gnlse_impl.h"
+#include "ofx_gnlse_wide.h"
 
 namespace ofx {
 
@@ -26,9 +27,34 @@ __global__ void __launch_bounds__(512) gnlse_kernel(GnlseArgs a) {
   gnlse_instance<R>(a, blockIdx.x, l0, l1, tw, red);
 }
 
+// n = 2^LG points, n / 8 threads (ofx_gnlse_wide.h)
+template <typename R, int LG>
+__global__ void __launch_bounds__((1 << LG) / GW_P) gnlse_wide_kernel(GnlseArgs a) {
+  extern __shared__ __align__(16) unsigned char gnlse_smem[];
+  cpx<R>* buf = reinterpret_cast<cpx<R>*>(gnlse_smem);
+  cpx<R>* tw = buf + gw_pad(1 << LG);
+  __shared__ double red[16];
+  GwThread<R> thr;
+  GwRun<R, LG> run;
+  run.thr = &thr;
+  run.red = red;
+  run.integrate(a, blockIdx.x, buf, tw);
+}
+
 }  // namespace ofx
 
 namespace {
+
+// the wide kernel for 2^lg points, or null where the general one runs
+template <typename R>
+const void* wide_kernel(int lg) {
+  if (!ofx::gw_runs(lg, sizeof(R) == 8)) return nullptr;
+  if constexpr (sizeof(R) == 8)
+    return lg == 11 ? (const void*)ofx::gnlse_wide_kernel<double, 11>
+                    : (const void*)ofx::gnlse_wide_kernel<double, 12>;
+  else
+    return (const void*)ofx::gnlse_wide_kernel<float, 13>;
+}
 
 struct DBuf {
   void* p = nullptr;
@@ -52,8 +78,9 @@ int gnlse_run(int n_inst, int n, int lg, int nsaves, const double* zs, const dou
               const double* fr, const double* dT, double rtol, double atol, long long max_steps,
               double* out, long long* stats, double* ms) {
   typedef ofx::cpx<R> C;
+  const void* wide = wide_kernel<R>(lg);
   // the FFT passes' twiddles, built in FP64 and rounded once
-  const std::vector<C> tw = ofx::fft_twiddles<R>(lg);
+  const std::vector<C> tw = wide ? ofx::gw_twiddles<R>(lg) : ofx::fft_twiddles<R>(lg);
   const size_t ni = (size_t)n_inst, nn = (size_t)n;
   std::vector<double> hB, hlre;
   std::vector<R> hW;
@@ -95,19 +122,21 @@ int gnlse_run(int n_inst, int n, int lg, int nsaves, const double* zs, const dou
   a.y0 = (const double*)b_y0.p;
   a.out = (double*)b_out.p;
   a.stats = (long long*)b_st.p;
-  // threads: a quarter of the points (one radix-4 butterfly each), 64..512
-  const int nt = std::min(512, std::max(64, n / 4));
-  const size_t lds = (2 * nn + tw.size()) * sizeof(C) + 8 * (size_t)(nt / 64);
-  st = hip_ok(hipFuncSetAttribute((const void*)ofx::gnlse_kernel<R>,
-                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  // threads: 8 points each in the wide kernel, else a quarter of the points
+  // (one radix-4 butterfly each), 64..512
+  const int nt = wide ? n / GW_P : std::min(512, std::max(64, n / 4));
+  const size_t lds = wide ? (ofx::gw_pad(n) + tw.size()) * sizeof(C)
+                          : (2 * nn + tw.size()) * sizeof(C) + 8 * (size_t)(nt / 64);
+  const void* kernel = wide ? wide : (const void*)ofx::gnlse_kernel<R>;
+  st = hip_ok(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   if (st) return st;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   if (!st) st = hip_ok(hipEventCreate(&e0));
   if (!st) st = hip_ok(hipEventCreate(&e1));
   if (!st) st = hip_ok(hipEventRecord(e0, 0));
   if (!st) {
-    hipLaunchKernelGGL(ofx::gnlse_kernel<R>, dim3(n_inst), dim3(nt), lds, 0, a);
-    st = hip_ok(hipGetLastError());
+    void* args[] = {&a};
+    st = hip_ok(hipLaunchKernel(kernel, dim3(n_inst), dim3(nt), args, lds, 0));
   }
   if (!st) st = hip_ok(hipEventRecord(e1, 0));
   if (!st) st = hip_ok(hipEventSynchronize(e1));

@@ -9,8 +9,24 @@
 
 #include "../../include/optifax_hip.h"
 #include "../../optifax_amd/csrc/ofx_gnlse_impl.h"
+#include "../../optifax_amd/csrc/ofx_gnlse_wide.h"
 
 namespace {
+
+// the wide kernel's instance (n / 8 threads, walked phase by phase)
+template <typename R, int LG>
+void run_wide(const ofx::GnlseArgs& a, int i) {
+  typedef ofx::cpx<R> C;
+  std::vector<C> buf(ofx::gw_pad(1 << LG)), tq(ofx::gw_table_size(LG)), tw = ofx::gw_twiddles<R>(LG);
+  ofx::GnlseArgs b = a;
+  b.tw = tw.data();
+  std::vector<ofx::GwThread<R>> thr((1 << LG) / GW_P);
+  double red[16];
+  ofx::GwRun<R, LG> r;
+  r.thr = thr.data();
+  r.red = red;
+  r.integrate(b, i, buf.data(), tq.data());
+}
 
 template <typename R>
 int run(int n_inst, int n, int lg, int nsaves, const double* zs, const double* y0,
@@ -47,7 +63,9 @@ int run(int n_inst, int n, int lg, int nsaves, const double* zs, const double* y
   a.stats = stats;
   std::vector<std::thread> th;
   for (int i = 0; i < n_inst; i++)
-    th.emplace_back([&a, &tw, i, n]() {
+    th.emplace_back([&a, &tw, i, n, lg]() {
+      if (ofx::gw_runs(lg, sizeof(R) == 8))
+        return lg == 11 ? run_wide<R, 11>(a, i) : lg == 12 ? run_wide<R, 12>(a, i) : run_wide<R, 13>(a, i);
       std::vector<C> l0(n), l1(n), tq(tw.size() + 1);
       double red[16];
       ofx::gnlse_instance<R>(a, i, l0.data(), l1.data(), tq.data(), red);
