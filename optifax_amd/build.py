@@ -8,6 +8,8 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -22,7 +24,8 @@ HIP_FLAGS = [
 ]
 
 LIB_SOURCES = ["ofx_backend_hip.hip", "ofx_backend_rkl.hip", "ofx_backend_wave.hip",
-               "ofx_runtime.cpp", "ofx_mlp.hip", "ofx_qpm.hip", "ofx_gnlse.hip"]
+               "ofx_backend_wave_fixed.hip", "ofx_runtime.cpp", "ofx_mlp.hip", "ofx_qpm.hip",
+               "ofx_gnlse.hip"]
 
 
 def _run(cmd):
@@ -38,8 +41,13 @@ def build_hip(verbose=False) -> str:
     os.makedirs(LIBDIR, exist_ok=True)
     out = os.path.join(LIBDIR, "libofx_hip.so")
     tmp = out + ".tmp"
-    cmd = [HIPCC, *HIP_FLAGS, "-shared", *[os.path.join(CSRC, s) for s in LIB_SOURCES], "-o", tmp]
-    log = _run(cmd)
+    with tempfile.TemporaryDirectory() as objdir:
+        objs = [os.path.join(objdir, s + ".o") for s in LIB_SOURCES]
+        cmds = [[HIPCC, *HIP_FLAGS, "-c", os.path.join(CSRC, s), "-o", o]
+                for s, o in zip(LIB_SOURCES, objs)]
+        with ThreadPoolExecutor(len(cmds)) as pool:
+            log = "\n".join(pool.map(_run, cmds))
+        log += _run([HIPCC, HIP_FLAGS[0], "-shared", *objs, "-o", tmp])
     if verbose and log.strip():
         print(log)
     os.replace(tmp, out)

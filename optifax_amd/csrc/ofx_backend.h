@@ -11,8 +11,15 @@
 enum { XMODE_RK23_LDS = 2 };
 // Bits 4..6: the wave kernel (ofx_wave_impl.h) with this many points a thread
 // (1, 2 or 4); bit 7: its form for workgroups of more than 256 threads.  The
-// other bits are then 0.
-enum { XMODE_WAVE_SHIFT = 4, XMODE_WAVE_MASK = 0x70, XMODE_WAVE_WIDE = 0x80 };
+// other bits are then 0.  Bits 8..12 instead: the wave kernel with the default
+// geometry of a grid of 2^that many points fixed.
+enum {
+  XMODE_WAVE_SHIFT = 4,
+  XMODE_WAVE_MASK = 0x70,
+  XMODE_WAVE_WIDE = 0x80,
+  XMODE_FIXED_SHIFT = 8,
+  XMODE_FIXED_MASK = 0x1f00
+};
 
 namespace ofx {
 

@@ -28,10 +28,15 @@ __global__ void __launch_bounds__(512) pass_kernel(LaunchArgs a) {
 const void* rkl_kernel(int precision, int xmode);
 // the wave kernels (ofx_backend_wave.hip)
 const void* wave_kernel_fn(int precision, int points, bool wide);
+// the same with a grid size's default geometry fixed (ofx_backend_wave_fixed.hip)
+const void* wave_fixed_fn(int precision, int lg);
 
 // the kernel instantiation for a precision and xmode (exchange mode in bit 0,
-// XMODE_RK23_LDS in bit 1, the wave kernel's points a thread in bits 4..6)
+// XMODE_RK23_LDS in bit 1, the wave kernel's points a thread in bits 4..6, its
+// fixed grid size in bits 8..12)
 static const void* pass_fn(int precision, int xmode) {
+  if (xmode & XMODE_FIXED_MASK)
+    return wave_fixed_fn(precision, (xmode & XMODE_FIXED_MASK) >> XMODE_FIXED_SHIFT);
   if (xmode & XMODE_WAVE_MASK)
     return wave_kernel_fn(precision, (xmode & XMODE_WAVE_MASK) >> XMODE_WAVE_SHIFT,
                           (xmode & XMODE_WAVE_WIDE) != 0);
@@ -154,6 +159,10 @@ int be_create(int device, Backend** out, DeviceInfo* info) {
                      4 << XMODE_WAVE_SHIFT | XMODE_WAVE_WIDE})
         ok = ok && hipFuncSetAttribute(pass_fn(prec, xm), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        dyn) == hipSuccess;
+    for (int prec : {OFX_F32, OFX_F64})
+      for (int lg = WAVE_FIXED_LG; lg <= 16; lg++)
+        ok = ok && hipFuncSetAttribute(pass_fn(prec, lg << XMODE_FIXED_SHIFT),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, dyn) == hipSuccess;
     if (!ok)
       snprintf(info->name + strlen(info->name), sizeof info->name - strlen(info->name),
                " [dyn-LDS attribute not set]");

@@ -1,5 +1,6 @@
 // The wave kernels (ofx_wave_impl.h): the Heun pass and round trip with small
-// shares per workgroup, by precision and points a thread.
+// shares per workgroup, by precision and points a thread, for any geometry
+// (default geometries: ofx_backend_wave_fixed.hip).
 #include <hip/hip_runtime.h>
 
 #include "../../include/optifax_hip.h"
@@ -17,7 +18,8 @@ __global__ void __launch_bounds__(MAXT) wave_kernel(LaunchArgs a) {
   __shared__ double red[64];
   __shared__ int sflag[4];
   WvThread<R, S> thr;
-  wave_main<R, S>(a, (int)blockIdx.x, reinterpret_cast<cpx<R>*>(ofx_lds_raw), red, sflag, &thr);
+  wave_main<R, S, WvGeoRt, sizeof(R) == 8 || (MAXT > 256)>(
+      a, (int)blockIdx.x, reinterpret_cast<cpx<R>*>(ofx_lds_raw), red, sflag, &thr);
 }
 
 template <typename R, int MAXT>

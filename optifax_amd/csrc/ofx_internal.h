@@ -21,6 +21,36 @@ enum {
   ST_BAD_ARG = 5,
 };
 
+// Default geometry of the wave kernel (ofx_wave_impl.h) on a grid of 2^lg
+// points, lg <= 16: log2 of the workgroups an instance and the threads of each.
+// For lg >= WAVE_FIXED_LG a kernel with this geometry fixed exists; smaller
+// grids are not used in earnest.  us per adaptive step, FP32 / FP64, of one
+// instance by workgroups (each with its best thread count, all with the
+// geometry fixed); the general kernel at its best geometry after the colon:
+//   2^8   1 workgroup 2.6 / 3.0, 4: 4.3 / 6.0
+//   2^9   1: 3.4 / 4.0, 8: 4.8 / 6.8                      : 7.9 / 8.9
+//   2^10  1: 4.1 / 6.0, 8: 4.9 / 6.8, 32: 5.3 / 7.9       : 8.7 / -
+//   2^11  8: 5.1 / 8.0, 16: 4.7 / 7.2, 32: 5.1 / 7.1      : 9.0 / 10.6
+//   2^12  16: 5.3 / 7.5, 32: 5.9 / 8.3                    : 10.2 / 11.7
+//   2^13  16: 6.8 / 10.7, 32: 6.2 / 9.9, 64: 7.3 / 11.3   : 11.0 / 12.8
+//   2^14  32: 8.1 / 12.6, 64: 7.2 / 9.9, 128: 7.3 / 10.5  : 12.2 / 14.5
+//   2^15  64: 8.1 / 11.9, 128: 8.0 / 11.1                 : 12.7 / 16.1
+//   2^16  64: 12.2 / 17.3, 128: 10.2 / 15.5               : 15.4 / -
+// Threads: 4 transform elements each where that leaves the stages at most 2
+// points a thread (2^12 FP32 at 16 workgroups: 128 threads 6.3, 256 5.3; 2^15
+// at 128: 128 threads 9.9, 256 8.0, 512 10.2).
+enum { WAVE_FIXED_LG = 8 };
+struct WaveGeometry {
+  int lgC, block;
+};
+constexpr WaveGeometry wave_geometry(int lg, bool f64) {
+  return lg <= 10   ? WaveGeometry{0, lg < 6 ? 64 : lg < 8 ? 1 << lg : lg < 10 || f64 ? 256 : 512}
+         : lg == 11 ? WaveGeometry{4, 128}
+         : lg == 12 ? WaveGeometry{4, 256}
+         : lg <= 14 ? WaveGeometry{lg - 8, 256}
+                    : WaveGeometry{7, lg == 16 && !f64 ? 512 : 256};
+}
+
 // Everything one instance needs on the device.  One array entry per instance,
 // uploaded once per run; pointers are device pointers.
 struct InstDesc {
@@ -93,11 +123,11 @@ struct LaunchArgs {
   const int* wg_rank;      // per workgroup: rank within its cluster
   const void* twiddle;     // NMAX complex: exp(-2 pi i m / NMAX)
   int nmax;                // twiddle table size (largest N in the launch)
-  int block;               // threads per workgroup
   int trips;               // 0: single pass (MEX mode); >0: round trips
   double conv_tol;         // stop an instance when conv metric < tol (<=0 never)
   unsigned long long timeout_ticks;  // barrier spin limit in wall-clock ticks
   int* xcc_ids;            // optional: per workgroup hardware XCC id (diagnostic)
+  int block;               // threads per workgroup
 };
 
 }  // namespace ofx

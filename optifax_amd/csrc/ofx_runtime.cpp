@@ -129,6 +129,12 @@ size_t lds_bytes_for(int n1, int n2, int C, int method, size_t csz) {
           ((size_t)W * (size_t)n2 + 1) / 2) * csz + 16 + (size_t)(n1 + n2) * 16;
 }
 
+// largest cluster size the method allows (RK23 exchanges 3 boundary columns
+// of K4 with each neighbour, so each workgroup owns at least 4 columns)
+int max_cluster(int method, int n1, int n2) {
+  return method == OFX_METHOD_RK23 ? std::min(n1 / 4, n2) : std::min(n1, n2);
+}
+
 // LDS of a workgroup of the wave kernel: A0 with its halo, the column slots
 // (272 elements each 256) and the row slots (ofx_wave_impl.h)
 size_t wave_lds_bytes(int n1, int n2, int C, size_t csz) {
@@ -150,31 +156,17 @@ int wave_points(const ofx_pass_params& p, int n1, int C, int block, size_t csz, 
 
 // Workgroups per instance for the wave kernel, or 0 when it does not apply.
 // A grid of up to 2^10 points runs in one workgroup without any exchange; a
-// larger one takes the workgroups that measured fastest (us per adaptive
-// step, FP32 / FP64, one instance; the general kernel at its best geometry
-// after the colon):
-//   2^9   1 workgroup 5.5 / 6.1, 8: 6.8 / 7.6            : 7.9 / 8.9
-//   2^10  1: 6.5 / 7.9, 16: 7.5 / 8.1                    : 8.7 / -
-//   2^11  1: 8.4 / 15.8, 16: 7.5 / 8.6, 32: 7.3 / 8.2    : 9.0 / 10.6
-//   2^12  16: 8.3 / 10.2, 32: 8.1 / 10.5                 : 10.2 / 11.7
-//   2^13  16: 9.4 / 11.9, 32: 9.1 / 11.8                 : 11.0 / 12.8
-//   2^14  32: 10.6 / 14.8, 64: 9.2 / 11.8, 128: 9.9 / 12.6 : 12.2 / 14.5
-//   2^15  64: 10.0 / 12.9, 128: 10.0 / 13.7              : 12.7 / 16.1
-//   2^16  64: 12.4 / 18.6, 128: 12.0 / 17.7              : 15.4 / -
-// With several instances each takes what keeps them all resident, down to 4
-// points a thread of 256 (2^14 at 16 workgroups: 11.3 against 16.5).
-int wave_cluster(const ofx_pass_params& p, int n1, int n_inst, int cus) {
+// larger one takes the workgroups that measured fastest (wave_geometry).  With
+// several instances each takes what keeps them all resident, down to 4 points a
+// thread of 256 (2^14 at 16 workgroups: 11.3 us per step against the general
+// kernel's 16.5).
+int wave_cluster(const ofx_pass_params& p, int n1, int n_inst, int cus, size_t csz) {
   const int n = p.n;
   if (p.method != OFX_METHOD_HEUN || n1 > 256 || n / n1 > 256) return 0;
-  int C = n <= 1024 ? 1 : n <= 8192 ? 32 : n <= 16384 ? 64 : 128;
+  int C = 1 << wave_geometry(ilog2i(n), csz == 16).lgC;
   while (C > 1 && (long long)n_inst * C > cus) C >>= 1;
-  return n / C <= 1024 && (long long)n_inst * C <= cus ? C : 0;
-}
-
-// largest cluster size the method allows (RK23 exchanges 3 boundary columns
-// of K4 with each neighbour, so each workgroup owns at least 4 columns)
-int max_cluster(int method, int n1, int n2) {
-  return method == OFX_METHOD_RK23 ? std::min(n1 / 4, n2) : std::min(n1, n2);
+  const bool fits = n / C <= 1024 && (long long)n_inst * C <= cus;
+  return fits && C <= max_cluster(p.method, n1, n / n1) ? C : 0;
 }
 
 int dev_alloc(ofx_opo* r, void** p, size_t bytes) {
@@ -312,7 +304,7 @@ int plan_instance(ofx_context* ctx, const ofx_pass_params& p, int n_inst, const 
         (int)lds_bytes_for(n1, n2, C, meth, csz) > ctx->info.lds_max - 1024)
       return fail(ctx, OFX_E_ARG, "cluster size %d is invalid for N=%d (n1=%d)", C, n, n1);
   } else if (const int Cw = tune && tune->exchange == 2 ? 0
-                            : wave_cluster(p, n1, n_inst, ctx->info.cus)) {
+                            : wave_cluster(p, n1, n_inst, ctx->info.cus, csz)) {
     C = Cw;
   } else {
     // The general kernel: spread a small batch over more workgroups until a
@@ -329,18 +321,32 @@ int plan_instance(ofx_context* ctx, const ofx_pass_params& p, int n_inst, const 
   return OFX_OK;
 }
 
-// Threads per workgroup of the wave kernel for one instance: a wave for each
-// 256 elements of the own and halo columns (the step's longest transform
-// phase), 256 in a cluster of one for the stages' sake; at most 512 with FP32
-// fields (N = 2^16 at 128 workgroups: 12.0 us per step with 512 threads, 13.2
-// with 256) and 256 with FP64 fields (whose 512-thread form spills: 36 against
-// 17.7).  0 when the wave kernel cannot run the instance.
+// Threads per workgroup of the wave kernel for one instance: the default
+// geometry's where the cluster is its, else a wave for each 256 elements of the
+// own and halo columns (the step's longest transform phase), 256 in a cluster
+// of one for the stages' sake; at most 512 with FP32 fields (2^16 at 64
+// workgroups: 12.2 us per step with 512 threads, 12.7 with 256) and 256 with
+// FP64 fields (whose 512-thread form spills: 26 against 17.3).  0 when the wave
+// kernel cannot run the instance.
 int wave_block(const ofx_pass_params& p, int n1, int C, size_t csz, int lds_max) {
   const int n2 = p.n / n1, el = C == 1 ? p.n : (n1 / C + 4) * n2;
+  const WaveGeometry g = wave_geometry(ilog2i(p.n), csz == 16);
   int block = 64;
   while (block < el / 4 || block < n2 || (C == 1 && block < std::min(p.n, 256))) block <<= 1;
-  block = std::min(block, csz == 8 ? 512 : 256);
-  return wave_points(p, n1, C, block, csz, lds_max) ? block : 0;
+  block = C == 1 << g.lgC ? g.block : std::min(block, csz == 8 ? 512 : 256);
+  return p.n / C <= 1024 && wave_points(p, n1, C, block, csz, lds_max) ? block : 0;
+}
+
+// Launch mode of the wave kernel with this many points a thread (wave_points):
+// the kernel with the default geometry fixed where this is it for every
+// instance (2^8 2.6 against 4.1 us per step, 2^12 5.8 against 7.3, 2^15 8.1
+// against 9.2; FP64 2^15 11.0 against 13.4), else the one for any geometry.
+// lg: log2 of the common grid size of the instances, or 0.
+int wave_mode(int points, int block, int lg, int n1, int C, size_t csz) {
+  const WaveGeometry g = wave_geometry(lg, csz == 16);
+  if (lg >= WAVE_FIXED_LG && n1 == 1 << ((lg + 1) / 2) && C == 1 << g.lgC && block == g.block)
+    return lg << XMODE_FIXED_SHIFT;
+  return (points << XMODE_WAVE_SHIFT) | (block > 256 ? XMODE_WAVE_WIDE : 0);
 }
 
 // Threads per workgroup: the wave kernel's when it can run every instance
@@ -474,16 +480,22 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
     cmin = std::min(cmin, r->inst_C[i]);
   }
   r->xmode = exchange_mode(exchange, cmin);
-  // the wave kernel when it can run every instance
+  // the wave kernel when it suits every instance (a caller that asks for the
+  // tagged exchange has it wherever it can run)
   int points = 0;
-  for (int i = 0; i < n_inst && exchange != 2; i++) {
+  for (int i = 0; i < n_inst && (exchange == 1 || (exchange == 0 && wblock)); i++) {
     const int w = wave_points(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->block, r->csz,
                               ctx->info.lds_max);
     points = w ? std::max(points, w) : 0;
     if (!w) break;
   }
   if (points) {
-    r->xmode = (points << XMODE_WAVE_SHIFT) | (r->block > 256 ? XMODE_WAVE_WIDE : 0);
+    bool same = true;  // one grid size and geometry throughout
+    for (int i = 1; i < n_inst; i++)
+      same = same && specs[i].pass.n == specs[0].pass.n && r->inst_n1[i] == r->inst_n1[0] &&
+             r->inst_C[i] == r->inst_C[0];
+    r->xmode = wave_mode(points, r->block, same ? ilog2i(specs[0].pass.n) : 0, r->inst_n1[0],
+                         r->inst_C[0], r->csz);
     lds = 0;
     for (int i = 0; i < n_inst; i++)
       lds = std::max(lds, wave_lds_bytes(r->inst_n1[i], specs[i].pass.n / r->inst_n1[i],
@@ -1238,13 +1250,12 @@ extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params*
   // cluster per instance, all resident at once)
   int C = 0, n1 = 0, block = 0;
   st = plan_instance(ctx, *p, batch, nullptr, 0, 0, 8, &C, &n1);
-  if (!st)
-    st = plan_block(ctx, nullptr, C, wave_block(*p, n1, C, 8, ctx->info.lds_max), &block);
+  const int wblock = st ? 0 : wave_block(*p, n1, C, 8, ctx->info.lds_max);
+  if (!st) st = plan_block(ctx, nullptr, C, wblock, &block);
   if (st) return st;
   const int n2 = n / n1;
-  const int points = wave_points(*p, n1, C, block, 8, ctx->info.lds_max);
-  const int xmode = points ? (points << XMODE_WAVE_SHIFT) | (block > 256 ? XMODE_WAVE_WIDE : 0)
-                           : exchange_mode(0, C);
+  const int points = wblock ? wave_points(*p, n1, C, block, 8, ctx->info.lds_max) : 0;
+  const int xmode = points ? wave_mode(points, block, ilog2i(n), n1, C, 8) : exchange_mode(0, C);
   const size_t lds = points ? wave_lds_bytes(n1, n2, C, 8) : lds_bytes_for(n1, n2, C, method, 8);
   const int bpc = be_blocks_per_cu(ctx->be, OFX_F32, xmode, block, lds);
   if (bpc < 1)

@@ -25,10 +25,13 @@
 // form none.
 //
 // Bound: the latency of the step's dependent chain (two exchanges of ~1 us
-// each way plus about 20 LDS round trips), not arithmetic or memory.  One
-// instance, us per adaptive step, FP32, against the general kernel at its
-// best geometry: 2^9 points 5.4 (7.9), 2^11 7.3 (9.0), 2^13 9.1 (11.0), 2^15
-// 10.0 (12.7), 2^16 12.0 (15.4); FP64 2^14 11.8 (14.5).
+// each way plus about 20 LDS round trips, and 5 to 8 cycles for each
+// instruction of a wave that is alone on its SIMD), not arithmetic or memory.
+// With the geometry a compile-time constant (WvGeoCt) index arithmetic, address
+// registers and the branches on it go.  One instance, us per adaptive step,
+// FP32, against the general kernel at its best geometry: 2^9 points 3.4 (7.9),
+// 2^11 4.7 (9.0), 2^13 6.2 (11.0), 2^15 8.0 (12.7), 2^16 10.2 (15.4); FP64 2^14
+// 9.9 (14.5).
 #pragma once
 #include "ofx_pass_impl.h"
 
@@ -79,6 +82,12 @@ OFX_DEV cpx<R> wv_mulq(cpx<R> a, cpx<R> b) {
 template <typename R>
 OFX_DEV cpx<R> wv_mulc(cpx<R> a, cpx<R> b) {
   return mkc<R>(wv_fma(a.x, b.x, a.y * b.y), wv_fma(a.y, b.x, -(a.x * b.y)));
+}
+// |a|^2 in FP64
+template <typename R>
+OFX_DEV double wv_abs2(cpx<R> a) {
+  const double x = a.x, y = a.y;
+  return wv_fma(x, x, y * y);
 }
 // nl_term_e
 template <typename R>
@@ -144,6 +153,29 @@ OFX_DEV void wv_r4(cpx<R>* v, const cpx<R>* w) {
 OFX_DEV int wv_exchanges(int lg) { return (lg & 1) ? (lg - 1) >> 1 : (lg >> 1) - 1; }
 OFX_DEV int wv_stride(int lg, int e) { return (lg & 1) ? 2 << (2 * e) : 4 << (2 * e); }
 
+// A tagged element's place: words at base + i ws (uniform) plus a 32-bit byte
+// offset of the lane, so that an access needs no 64-bit lane address.
+struct WvAt {
+  const u64* base;
+  size_t ws;
+  unsigned off;
+};
+template <typename T>
+OFX_DEV void wv_load(const WvAt& t, u64* w) {
+#pragma unroll
+  for (int i = 0; i < Tagged<T>::NW; i++)
+    w[i] = tag_load((const u64*)((const char*)(t.base + i * t.ws) + t.off));
+}
+template <typename T>
+OFX_DEV void wv_put(const WvAt& t, T v, unsigned tag) {
+  typedef Tagged<T> TT;
+  const typename TT::Words x = __builtin_bit_cast(typename TT::Words, v);
+  const u64 hi = (u64)tag << 32;
+#pragma unroll
+  for (int i = 0; i < TT::NW; i++)
+    tag_store((u64*)((char*)const_cast<u64*>(t.base + i * t.ws) + t.off), hi | (u64)x.w[i]);
+}
+
 // Poll `N` tagged elements of this thread (those of `mask`): loads are issued
 // together, repeated for the words that are still old, and the clock and the
 // abort flag are looked at while a repeat is in flight.
@@ -155,8 +187,7 @@ OFX_DEV bool wv_poll(unsigned mask, unsigned tag, Src src, Commit commit, Spin& 
 #pragma unroll
   for (int j = 0; j < N; j++)
     if ((pend >> j) & 1u) {
-      const TagPtr t = src(j);
-      TT::load(t.p, t.ws, 0, tag, w[j]);
+      wv_load<T>(src(j), w[j]);
     }
   for (;;) {
 #pragma unroll
@@ -169,8 +200,7 @@ OFX_DEV bool wv_poll(unsigned mask, unsigned tag, Src src, Commit commit, Spin& 
 #pragma unroll
     for (int j = 0; j < N; j++)
       if ((pend >> j) & 1u) {
-        const TagPtr t = src(j);
-        TT::load(t.p, t.ws, 0, tag, w[j]);
+        wv_load<T>(src(j), w[j]);
       }
 #ifdef OFX_EMU
     sched_yield();
@@ -214,12 +244,49 @@ OFX_DEV double wv_wave_max(double v) {
 }
 #endif
 
+// Launch geometry of a member: read from the instance and the launch ...
+struct WvGeoRt {
+  static constexpr bool FIXED = false;
+  int n, n1, n2, lg1, lg2, lgW, Cn, W, Rr, LC, sT, NT, nw;
+  OFX_DEV void set(const InstDesc& d, int C, int block) {
+    n = d.n;
+    n1 = d.n1;
+    n2 = d.n2;
+    lg1 = d.lg1;
+    lg2 = d.lg2;
+    Cn = C;
+    int lgC = 0;
+    while ((1 << lgC) < C) lgC++;
+    W = n1 >> lgC;
+    lgW = lg1 - lgC;
+    Rr = n2 >> lgC;
+    LC = W + 4;
+    sT = n2 + 1;
+    NT = block;
+    nw = NT >> 6;
+  }
+};
+// ... or fixed for a grid size's default geometry: shifts, strides, slot and
+// wave counts are then constants (about half of a step's instructions form
+// indices otherwise).
+template <int LG, int LGC, int NT_>
+struct WvGeoCt {
+  static constexpr bool FIXED = true;
+  static constexpr int n = 1 << LG, lg1 = (LG + 1) / 2, lg2 = LG - lg1, n1 = 1 << lg1, n2 = 1 << lg2,
+                       Cn = 1 << LGC, W = n1 >> LGC, lgW = lg1 - LGC, Rr = n2 >> LGC, LC = W + 4,
+                       sT = n2 + 1, NT = NT_, nw = NT >> 6;
+  OFX_DEV void set(const InstDesc&, int, int) {}
+};
+
 // One member's share of one instance.
-template <typename R, int S>
-struct WvRun {
+template <typename R, int S, typename GEO, bool REFRESH>
+struct WvRun : GEO {
   typedef cpx<R> C;
   typedef Tagged<C> TT;
   typedef WvThread<R, S> T;
+  using GEO::n; using GEO::n1; using GEO::n2; using GEO::lg1; using GEO::lg2; using GEO::lgW;
+  using GEO::Cn; using GEO::W; using GEO::Rr; using GEO::LC; using GEO::sT; using GEO::NT;
+  using GEO::nw;
   const LaunchArgs& a;
   const ClusterDesc& cd;
   const InstDesc& d;
@@ -227,8 +294,7 @@ struct WvRun {
   double* red;   // [0, 16) wave maxima, [32] the cluster's maximum
   int* sflag;    // [0] barrier verdict, [1] a poll gave up
   T* thr;
-  int rank, NT, nw, wv, tid;
-  int n, n1, n2, lg1, lg2, lgW, Cn, W, Rr, LC, sT, c0, k20;
+  int rank, wv, tid, c0, k20;
   C *A0, *X, *Tb;
   u64 *t1b, *t2b, *slots;
   int* abort_flag;
@@ -249,10 +315,14 @@ struct WvRun {
   }
   // Hides where the lane's indices come from, so that the addresses formed
   // from them are formed again in every step instead of being kept in
-  // registers across it (kept, they spill)
+  // registers across it.  Kept they are 10 % faster with a fixed geometry (2^15
+  // points 8.0 against 8.6 us per step) and, where they fit, with a run-time one
+  // (FP32 fields in workgroups of 256: 9.0 against 10.0); elsewhere they spill
+  // (FP64 14.6 against 13.4, 512 threads 18.9 against 11.9).
   OFX_DEV void refresh() {
 #ifndef OFX_EMU
-    asm volatile("" : "+v"(tid), "+v"(thr->jr), "+v"(thr->qr), "+v"(thr->jc), "+v"(thr->qc));
+    if constexpr (REFRESH)
+      asm volatile("" : "+v"(tid), "+v"(thr->jr), "+v"(thr->qr), "+v"(thr->jc), "+v"(thr->qc));
 #endif
   }
   // workgroup barrier (one wave needs none: only the order of its accesses)
@@ -441,7 +511,7 @@ struct WvRun {
         if (Cn == 1)
           Tb[wv_pad((k2 << lg1) + cl)] = v;
         else
-          TT::put(t1 + t1_at(c0 + cl, k2), (size_t)n, 0, v, tag);
+          wv_put<C>(WvAt{t1, (size_t)n, t1_at(c0 + cl, k2) * 8u}, v, tag);
       }
     });
   }
@@ -462,7 +532,7 @@ struct WvRun {
         if (Cn == 1)
           X[wv_pad((c << lg2) + rl)] = v;
         else
-          TT::put(t2 + (unsigned)(((k20 + rl) << lg1) + c), (size_t)n, 0, v, tag);
+          wv_put<C>(WvAt{t2, (size_t)n, (unsigned)(((k20 + rl) << lg1) + c) * 8u}, v, tag);
       }
     });
   }
@@ -494,9 +564,9 @@ struct WvRun {
       Spin sp = spin();
       ok = wv_poll<C, 6>(
                mask, tag,
-               [&](int j) -> TagPtr {
-                 if (j < 4) return TagPtr{t1 + t1_at(t.jr + l4 * j, k20 + rl), (size_t)n, 0};
-                 return TagPtr{record_of(x, lane + 64 * (j - 4)), 1, 0};
+               [&](int j) -> WvAt {
+                 if (j < 4) return WvAt{t1, (size_t)n, t1_at(t.jr + l4 * j, k20 + rl) * 8u};
+                 return WvAt{record_of(x, 0), 1, (unsigned)((lane + 64 * (j - 4)) * TT::NW) * 8u};
                },
                [&](int j, C c) {
                  if (j < 4)
@@ -576,7 +646,7 @@ struct WvRun {
           }
         }
         ok = wv_poll<C, 4>(
-            mask, tag, [&](int b) { return TagPtr{t2 + src[b], (size_t)n, 0}; },
+            mask, tag, [&](int b) { return WvAt{t2, (size_t)n, src[b] * 8u}; },
             [&](int b, C v) { X[dst[b]] = v; }, sp);
       }
       if (!ok) sflag[1] = 1;
@@ -613,32 +683,18 @@ struct WvRun {
   OFX_DEV void run(int rank_, C* lds);
 };
 
-template <typename R, int S>
-OFX_DEV void WvRun<R, S>::run(int rank_, C* lds) {
+template <typename R, int S, typename GEO, bool REFRESH>
+OFX_DEV void WvRun<R, S, GEO, REFRESH>::run(int rank_, C* lds) {
   // converged in an earlier launch (and not rewritten since): nothing to do
   if (a.conv_tol > 0.0 && a.trips > 0 && d.status[0] == ST_CONVERGED) return;
   rank = rank_;
-  NT = a.block;
-  nw = NT >> 6;
 #ifdef OFX_EMU
   wv = tid = 0;
 #else
   tid = (int)threadIdx.x;
   wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
 #endif
-  n = d.n;
-  n1 = d.n1;
-  n2 = d.n2;
-  lg1 = d.lg1;
-  lg2 = d.lg2;
-  Cn = cd.C;
-  int lgC = 0;
-  while ((1 << lgC) < Cn) lgC++;
-  W = n1 >> lgC;
-  lgW = lg1 - lgC;
-  Rr = n2 >> lgC;
-  LC = W + 2 * HW;
-  sT = n2 + 1;
+  GEO::set(d, cd.C, a.block);
   c0 = rank * W;
   k20 = rank * Rr;
   t1b = (u64*)uniform(cd.t1);
@@ -752,7 +808,7 @@ OFX_DEV void WvRun<R, S>::run(int rank_, C* lds) {
         tag1 = sy.base + x1;
         each([&](int tid, int, T&) {
           if (tid == NT - 1)
-            TT::put(record_of(x1, rank), 1, 0, pack_d<R>(gmax), tag1);
+            wv_put<C>(WvAt{record_of(x1, rank), 1, 0u}, pack_d<R>(gmax), tag1);
         });
       }
       const bool early = Cn == 1;  // the decision needs no exchange
@@ -899,16 +955,16 @@ OFX_DEV void WvRun<R, S>::run(int rank_, C* lds) {
         for (int m = 0; m < 4; m++) {
           const int kk = (k20 + rl) + n2 * (t.jr + m * (n1 >> 2));
           const C v = t.v[m];
-          xesd[kk] += (double)v.x * (double)v.x + (double)v.y * (double)v.y;
+          xesd[kk] += wv_abs2(v);
           if (hist) hist[kk] = v;
           const C o = wv_mulq(v, ocm[kk]);
-          const double So = (double)o.x * (double)o.x + (double)o.y * (double)o.y;
+          const double So = wv_abs2(o);
           if (have_prev) {
             const C op = ocs[kk];
-            const double Sp = (double)op.x * (double)op.x + (double)op.y * (double)op.y;
-            acc[0] += (So - Sp) * (So - Sp);
+            const double Sp = wv_abs2(op);
+            acc[0] = wv_fma(So - Sp, So - Sp, acc[0]);
           }
-          acc[1] += So * So;
+          acc[1] = wv_fma(So, So, acc[1]);
           acc[2] += So;
           ocs[kk] = o;
           esd[kk] += So;
@@ -966,7 +1022,7 @@ OFX_DEV void WvRun<R, S>::run(int rank_, C* lds) {
   meet();  // (the next instance writes A0)
 }
 
-template <typename R, int S>
+template <typename R, int S, typename GEO, bool REFRESH>
 OFX_DEV void wave_main(const LaunchArgs& a, int wg, cpx<R>* lds, double* red, int* sflag,
                        WvThread<R, S>* thr) {
   const int ci = a.wg_cluster[wg];
@@ -977,7 +1033,7 @@ OFX_DEV void wave_main(const LaunchArgs& a, int wg, cpx<R>* lds, double* red, in
   member_begin(a, cd, wg, rank, sflag, sy);
   for (int ii = 0; ii < cd.n_inst; ii++) {
     const int id = a.inst_order[cd.first_inst + ii];
-    WvRun<R, S> run(a, cd, a.inst[id], sy, red, sflag, thr);
+    WvRun<R, S, GEO, REFRESH> run(a, cd, a.inst[id], sy, red, sflag, thr);
     run.run(rank, lds);
     if (flag_load(cd.abort_flag)) break;
   }

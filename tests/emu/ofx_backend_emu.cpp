@@ -98,11 +98,38 @@ static void run_wave(const LaunchArgs* a, int wg, size_t lds) {
   std::vector<WvThread<R, S>> thr((size_t)a->block);
   double red[64];
   int sflag[4];
-  wave_main<R, S>(*a, wg, reinterpret_cast<cpx<R>*>(mem.data()), red, sflag, thr.data());
+  wave_main<R, S, WvGeoRt, false>(*a, wg, reinterpret_cast<cpx<R>*>(mem.data()), red, sflag, thr.data());
 }
 template <typename R>
 static void (*wave_fn(int points))(const LaunchArgs*, int, size_t) {
   return points == 4 ? run_wave<R, 4> : points == 2 ? run_wave<R, 2> : run_wave<R, 1>;
+}
+
+// its forms with a fixed default geometry
+template <typename R, int LG>
+static void run_fixed(const LaunchArgs* a, int wg, size_t lds) {
+  constexpr WaveGeometry g = wave_geometry(LG, sizeof(R) == 8);
+  constexpr int share = (1 << LG) >> g.lgC, S = share > g.block ? share / g.block : 1;
+  std::vector<unsigned char> mem(lds + 64);
+  std::vector<WvThread<R, S>> thr((size_t)a->block);
+  double red[64];
+  int sflag[4];
+  wave_main<R, S, WvGeoCt<LG, g.lgC, g.block>, false>(
+      *a, wg, reinterpret_cast<cpx<R>*>(mem.data()), red, sflag, thr.data());
+}
+template <typename R>
+static void (*fixed_fn(int lg))(const LaunchArgs*, int, size_t) {
+  switch (lg) {
+    case 8: return run_fixed<R, 8>;
+    case 9: return run_fixed<R, 9>;
+    case 10: return run_fixed<R, 10>;
+    case 11: return run_fixed<R, 11>;
+    case 12: return run_fixed<R, 12>;
+    case 13: return run_fixed<R, 13>;
+    case 14: return run_fixed<R, 14>;
+    case 15: return run_fixed<R, 15>;
+    default: return run_fixed<R, 16>;
+  }
 }
 
 int be_launch(Backend* b, const LaunchArgs& a, int precision, int xmode, int grid, int block,
@@ -120,7 +147,10 @@ int be_launch(Backend* b, const LaunchArgs& a, int precision, int xmode, int gri
     std::vector<std::thread> th;
     const bool bar = (xmode & 1) == XM_BARRIER;
     for (int wg = 0; wg < grid; wg++) {
-      if (xmode & XMODE_WAVE_MASK) {
+      if (xmode & XMODE_FIXED_MASK) {
+        const int lg = (xmode & XMODE_FIXED_MASK) >> XMODE_FIXED_SHIFT;
+        th.emplace_back(precision == OFX_F64 ? fixed_fn<double>(lg) : fixed_fn<float>(lg), &a, wg, lds);
+      } else if (xmode & XMODE_WAVE_MASK) {
         const int pts = (xmode & XMODE_WAVE_MASK) >> XMODE_WAVE_SHIFT;
         th.emplace_back(precision == OFX_F64 ? wave_fn<double>(pts) : wave_fn<float>(pts), &a, wg, lds);
       } else if (xmode & XMODE_RK23_LDS)

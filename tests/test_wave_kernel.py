@@ -5,7 +5,8 @@ bits.
 
 Geometries: one workgroup without an exchange, one wave per workgroup, several
 waves, odd and even transform lengths on either side, a partly filled wave of
-rows and of columns, 1, 2 and 4 points a thread."""
+rows and of columns, 1, 2 and 4 points a thread; the default geometries, whose
+kernels have them fixed at compile time."""
 import os
 
 import numpy as np
@@ -18,6 +19,10 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 SMALL = [(64, 1, 64), (64, 2, 64), (128, 1, 64), (256, 1, 64), (256, 4, 64), (512, 8, 64),
          (512, 1, 128), (1024, 16, 64), (1024, 1, 256), (2048, 1, 512)]
 LARGE = [(4096, 32, 128), (8192, 32, 128), (16384, 64, 256), (32768, 128, 256), (65536, 128, 512)]
+
+FIXED_EMU = [(256, 1, 256), (512, 1, 256), (1024, 1, 512), (2048, 16, 128), (4096, 16, 256)]
+FIXED = FIXED_EMU + [(8192, 32, 256)]
+FIXED_F64 = [(1024, 1, 256), (65536, 128, 256)]   # (where FP64's differ from FP32's)
 
 
 def both(ctx, n, C, block, precision, trips, length):
@@ -68,14 +73,14 @@ def emu():
 
 
 @pytest.mark.parametrize("precision", ["single", "double"])
-@pytest.mark.parametrize("n,C,block", SMALL)
+@pytest.mark.parametrize("n,C,block", SMALL + FIXED_EMU)
 def test_emulated_wave_kernel_matches_general(emu, n, C, block, precision):
     check(*both(emu, n, C, block, precision, 2, 6e-6))
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("precision", ["single", "double"])
-@pytest.mark.parametrize("n,C,block", SMALL + LARGE)
+@pytest.mark.parametrize("n,C,block", SMALL + LARGE + FIXED + FIXED_F64)
 def test_wave_kernel_matches_general(n, C, block, precision):
     ctx = Context(0)
     check(*both(ctx, n, C, block, precision, 2, 20e-6))
