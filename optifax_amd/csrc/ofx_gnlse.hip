@@ -27,34 +27,12 @@ __global__ void __launch_bounds__(512) gnlse_kernel(GnlseArgs a) {
   gnlse_instance<R>(a, blockIdx.x, l0, l1, tw, red);
 }
 
-// n = 2^LG points, n / 8 threads (ofx_gnlse_wide.h)
-template <typename R, int LG>
-__global__ void __launch_bounds__((1 << LG) / GW_P) gnlse_wide_kernel(GnlseArgs a) {
-  extern __shared__ __align__(16) unsigned char gnlse_smem[];
-  cpx<R>* buf = reinterpret_cast<cpx<R>*>(gnlse_smem);
-  cpx<R>* tw = buf + gw_pad(1 << LG);
-  __shared__ double red[16];
-  GwThread<R> thr;
-  GwRun<R, LG> run;
-  run.thr = &thr;
-  run.red = red;
-  run.integrate(a, blockIdx.x, buf, tw);
-}
+// the wide kernel for n = 2^lg points (ofx_gnlse_wide.hip)
+const void* gnlse_wide_fn(int precision, int lg);
 
 }  // namespace ofx
 
 namespace {
-
-// the wide kernel for 2^lg points, or null where the general one runs
-template <typename R>
-const void* wide_kernel(int lg) {
-  if (!ofx::gw_runs(lg, sizeof(R) == 8)) return nullptr;
-  if constexpr (sizeof(R) == 8)
-    return lg == 11 ? (const void*)ofx::gnlse_wide_kernel<double, 11>
-                    : (const void*)ofx::gnlse_wide_kernel<double, 12>;
-  else
-    return (const void*)ofx::gnlse_wide_kernel<float, 13>;
-}
 
 struct DBuf {
   void* p = nullptr;
@@ -78,7 +56,9 @@ int gnlse_run(int n_inst, int n, int lg, int nsaves, const double* zs, const dou
               const double* fr, const double* dT, double rtol, double atol, long long max_steps,
               double* out, long long* stats, double* ms) {
   typedef ofx::cpx<R> C;
-  const void* wide = wide_kernel<R>(lg);
+  const bool f64 = sizeof(R) == 8;
+  const void* wide =
+      ofx::gw_runs(lg, f64) ? ofx::gnlse_wide_fn(f64 ? OFX_F64 : OFX_F32, lg) : nullptr;
   // the FFT passes' twiddles, built in FP64 and rounded once
   const std::vector<C> tw = wide ? ofx::gw_twiddles<R>(lg) : ofx::fft_twiddles<R>(lg);
   const size_t ni = (size_t)n_inst, nn = (size_t)n;
