@@ -372,6 +372,137 @@ int exchange_mode(int exchange, int cmin) {
   return exchange == 1 ? 0 : exchange == 2 ? 1 : (cmin >= 64 ? 0 : 1);
 }
 
+// An adaptive step's time [us] on a full device, fitted (within 10 %) to full
+// devices of 2^12 to 2^16 points at 256 to 4096 points a workgroup: general
+// kernel FP32 2^12 15.8 us at 1024 points, 34.7 at 4096; 2^16 22 and 39; FP64
+// 2^12 19.5 at 1024, 2^15 33 at 2048; wave kernel FP32 2^12 9.1 at 512, 2^15
+// 14.6 at 1024, FP64 2^12 13.2 and 2^15 20.6.  Only ratios are used.
+double step_us(const ofx_pass_params& p, int C, bool f64, bool wave) {
+  const double x = ilog2i(p.n) - 14, share = (double)p.n / C;
+  if (wave) return f64 ? 13.6 + 1.3 * x + 4.5e-3 * share : 6.9 + 0.7 * x + 6.5e-3 * share;
+  const double t = f64 ? 13.0 + 1.2 * x + 9.2e-3 * share
+                       : 12.5 + 1.2 * x + 5.2e-3 * share + 1.7e-3 * std::max(0.0, share - 2048);
+  return p.method == OFX_METHOD_RK23 ? 1.2 * std::max(t, 4.0) : std::max(t, 4.0);
+}
+
+// Instances to clusters: a cluster runs its members one after the other.
+struct BatchPlan {
+  std::vector<int> C;                     // per instance
+  std::vector<std::vector<int>> members;  // per cluster
+  double span = 0.0;                      // estimated time of the longest cluster
+};
+
+// Equal shares: every instance keeps the cluster size C; groups of one grid,
+// split and method get clusters in proportion, filled longest first.
+BatchPlan plan_equal(int n_inst, const ofx_opo_spec* specs, const std::vector<int>& inst_C,
+                     const std::vector<int>& inst_n1, int slots, bool f64, bool wave) {
+  BatchPlan plan;
+  plan.C = inst_C;
+  std::map<std::tuple<int, int, int, int>, std::vector<int>> groups;
+  for (int i = 0; i < n_inst; i++)
+    groups[std::make_tuple(inst_C[i], specs[i].pass.n, inst_n1[i], specs[i].pass.method)]
+        .push_back(i);
+  long long want = 0;
+  for (auto& g : groups) want += (long long)std::get<0>(g.first) * (long long)g.second.size();
+  for (auto& g : groups) {
+    const int C = std::get<0>(g.first);
+    std::vector<int> ids = g.second;
+    long long ncl = (long long)ids.size();
+    if (want > slots) ncl = std::max(1LL, (long long)ids.size() * slots / want);
+    ncl = std::min(ncl, (long long)std::max(1, slots / C));
+    std::sort(ids.begin(), ids.end(), [&](int a, int b) {
+      const double ca = (double)specs[a].pass.nsteps, cb = (double)specs[b].pass.nsteps;
+      return ca != cb ? ca > cb : a < b;
+    });
+    std::vector<std::vector<int>> mem((size_t)ncl);
+    std::vector<double> load((size_t)ncl, 0.0);
+    for (int id : ids) {
+      size_t best = 0;
+      for (size_t c = 1; c < load.size(); c++)
+        if (load[c] < load[best]) best = c;
+      mem[best].push_back(id);
+      load[best] += (double)specs[id].pass.nsteps;
+    }
+    const double us = step_us(specs[ids[0]].pass, C, f64, wave);
+    for (size_t c = 0; c < mem.size(); c++) {
+      if (mem[c].empty()) continue;
+      plan.span = std::max(plan.span, load[c] * us);
+      plan.members.push_back(mem[c]);
+    }
+  }
+  return plan;
+}
+
+// Uneven shares: the shortest time within which every instance, on the fewest
+// workgroups that finish it in that time, finds a place in some cluster of its
+// size (first fit, longest first).  Few workgroups are the efficient choice (a
+// 2^16 step takes 39 us on 16 workgroups, 25 on 32); only what would outlast the
+// rest gets more.  Grids of different sizes may follow each other in a cluster:
+// an instance ends with a cluster barrier, and tags keep rising.  False if no
+// such plan exists.
+bool plan_uneven(int n_inst, const ofx_opo_spec* specs, const std::vector<int>& inst_n1, int cus,
+                 size_t csz, int lds_max, bool wave, BatchPlan* plan) {
+  const bool f64 = csz == 16;
+  struct Choice {
+    int C;
+    double t;
+  };
+  std::vector<std::vector<Choice>> can(n_inst);
+  double lo = 0.0;
+  for (int i = 0; i < n_inst; i++) {
+    const ofx_pass_params& p = specs[i].pass;
+    const int n1 = inst_n1[i], n2 = p.n / n1;
+    const int top = wave ? 1 << wave_geometry(ilog2i(p.n), f64).lgC : 128;
+    for (int C = 1; C <= std::min(std::min(max_cluster(p.method, n1, n2), top), cus); C <<= 1) {
+      if (wave ? !wave_block(p, n1, C, csz, lds_max)
+               : ((int)lds_bytes_for(n1, n2, C, p.method, csz) > lds_max - 1024 ||
+                  (C > 1 && p.n / C < 256)))
+        continue;
+      const double t = p.nsteps * step_us(p, C, f64, wave);
+      if (can[i].empty() || t < can[i].back().t) can[i].push_back({C, t});
+    }
+    if (can[i].empty()) return false;
+    lo = std::max(lo, can[i].back().t);
+  }
+  std::vector<int> order(n_inst);
+  std::vector<Choice> pick(n_inst);
+  for (double span = lo; span < lo * n_inst * 1.03; span *= 1.03) {
+    for (int i = 0; i < n_inst; i++) {
+      order[i] = i;
+      pick[i] = *std::find_if(can[i].begin(), can[i].end(), [&](const Choice& c) { return c.t <= span; });
+    }
+    std::sort(order.begin(), order.end(), [&](int a, int b) {
+      return pick[a].t != pick[b].t ? pick[a].t > pick[b].t : a < b;
+    });
+    std::map<std::pair<int, int>, std::vector<std::pair<double, std::vector<int>>>> bins;
+    long long used = 0;
+    for (int i : order) {
+      auto& of_size = bins[std::make_pair(pick[i].C, specs[i].pass.method)];
+      auto b = std::find_if(of_size.begin(), of_size.end(),
+                            [&](const auto& q) { return q.first + pick[i].t <= span; });
+      if (b == of_size.end()) {
+        used += pick[i].C;
+        if (used > cus) break;
+        b = of_size.insert(b, std::make_pair(0.0, std::vector<int>()));
+      }
+      b->first += pick[i].t;
+      b->second.push_back(i);
+    }
+    if (used > cus) continue;
+    plan->C.resize(n_inst);
+    plan->members.clear();
+    plan->span = 0.0;
+    for (int i = 0; i < n_inst; i++) plan->C[i] = pick[i].C;
+    for (auto& of_size : bins)
+      for (auto& b : of_size.second) {
+        plan->members.push_back(b.second);
+        plan->span = std::max(plan->span, b.first);
+      }
+    return true;
+  }
+  return false;
+}
+
 }  // namespace
 
 extern "C" {
@@ -460,92 +591,81 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
     }
   }
   r->nmax = nmax;
-  int cmin0 = 1 << 30, wblock = 0;
-  for (int i = 0; i < n_inst; i++) {
-    cmin0 = std::min(cmin0, r->inst_C[i]);
-    const int b = wave_block(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->csz, ctx->info.lds_max);
-    wblock = i && !wblock ? 0 : b ? std::max(wblock, b) : 0;
-  }
   const int exchange = tune ? tune->exchange : 0;
-  st = plan_block(ctx, tune, cmin0, wblock, &r->block);
+  bool given = n_inst < 2 || (tune && (tune->cluster || tune->block || tune->exchange));
+  bool all_rk23 = n_inst > 0;
+  for (int i = 0; i < n_inst; i++) {
+    given = given || specs[i].cluster;
+    all_rk23 = all_rk23 && specs[i].pass.method == OFX_METHOD_RK23;
+  }
+  // threads, launch mode and LDS for the cluster sizes in r->inst_C
+  int slots = 0;
+  auto geometry = [&]() -> int {
+    int cmin = 1 << 30, wblock = 0;
+    for (int i = 0; i < n_inst; i++) {
+      cmin = std::min(cmin, r->inst_C[i]);
+      const int b = wave_block(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->csz, ctx->info.lds_max);
+      wblock = i && !wblock ? 0 : b ? std::max(wblock, b) : 0;
+    }
+    if (int st = plan_block(ctx, tune, cmin, wblock, &r->block)) return st;
+    // the wave kernel when it suits every instance (a caller that asks for the
+    // tagged exchange has it wherever it can run)
+    int points = 0;
+    for (int i = 0; i < n_inst && (exchange == 1 || (exchange == 0 && wblock)); i++) {
+      const int w = wave_points(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->block, r->csz,
+                                ctx->info.lds_max);
+      points = w ? std::max(points, w) : 0;
+      if (!w) break;
+    }
+    bool same = true;  // one grid size and geometry throughout
+    r->lds = 0;
+    for (int i = 0; i < n_inst; i++) {
+      const int n = specs[i].pass.n, n1 = r->inst_n1[i], C = r->inst_C[i];
+      same = same && n == specs[0].pass.n && n1 == r->inst_n1[0] && C == r->inst_C[0];
+      r->lds = std::max(r->lds, points ? wave_lds_bytes(n1, n / n1, C, r->csz)
+                                       : lds_bytes_for(n1, n / n1, C, specs[i].pass.method, r->csz));
+    }
+    r->xmode = points ? wave_mode(points, r->block, same ? ilog2i(specs[0].pass.n) : 0, r->inst_n1[0],
+                                  r->inst_C[0], r->csz)
+                      : exchange_mode(exchange, cmin);
+    if (all_rk23) r->xmode |= XMODE_RK23_LDS;
+    const int bpc = be_blocks_per_cu(ctx->be, precision, r->xmode, r->block, r->lds);
+    if (bpc < 1)
+      return fail(ctx, OFX_E_ARG, "kernel cannot launch with block=%d and %zu bytes of LDS", r->block,
+                  r->lds);
+    slots = ctx->info.cus * bpc;
+    return OFX_OK;
+  };
+  const bool f64 = precision == OFX_F64;
+  auto wave_runs = [&] { return (r->xmode & (XMODE_WAVE_MASK | XMODE_FIXED_MASK)) != 0; };
+  st = geometry();
   if (st) {
     delete r;
     return st;
   }
-  size_t lds = 0;
-  int cmin = 1 << 30;
-  for (int i = 0; i < n_inst; i++) {
-    const int n1 = r->inst_n1[i], n2 = specs[i].pass.n / n1;
-    lds = std::max(lds, lds_bytes_for(n1, n2, r->inst_C[i], specs[i].pass.method, r->csz));
-    cmin = std::min(cmin, r->inst_C[i]);
-  }
-  r->xmode = exchange_mode(exchange, cmin);
-  // the wave kernel when it suits every instance (a caller that asks for the
-  // tagged exchange has it wherever it can run)
-  int points = 0;
-  for (int i = 0; i < n_inst && (exchange == 1 || (exchange == 0 && wblock)); i++) {
-    const int w = wave_points(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->block, r->csz,
-                              ctx->info.lds_max);
-    points = w ? std::max(points, w) : 0;
-    if (!w) break;
-  }
-  if (points) {
-    bool same = true;  // one grid size and geometry throughout
-    for (int i = 1; i < n_inst; i++)
-      same = same && specs[i].pass.n == specs[0].pass.n && r->inst_n1[i] == r->inst_n1[0] &&
-             r->inst_C[i] == r->inst_C[0];
-    r->xmode = wave_mode(points, r->block, same ? ilog2i(specs[0].pass.n) : 0, r->inst_n1[0],
-                         r->inst_C[0], r->csz);
-    lds = 0;
-    for (int i = 0; i < n_inst; i++)
-      lds = std::max(lds, wave_lds_bytes(r->inst_n1[i], specs[i].pass.n / r->inst_n1[i],
-                                         r->inst_C[i], r->csz));
-  }
-  r->lds = lds;
-  bool all_rk23 = n_inst > 0;
-  for (int i = 0; i < n_inst; i++) all_rk23 = all_rk23 && specs[i].pass.method == OFX_METHOD_RK23;
-  if (all_rk23) r->xmode |= XMODE_RK23_LDS;
-  const int bpc = be_blocks_per_cu(ctx->be, precision, r->xmode, r->block, lds);
-  if (bpc < 1) {
-    delete r;
-    return fail(ctx, OFX_E_ARG, "kernel cannot launch with block=%d and %zu bytes of LDS", r->block, lds);
-  }
-  const int slots = ctx->info.cus * bpc;
 
-  // ---- clusters: group instances by (C, n, n1, method); LPT over cost ----
-  std::map<std::tuple<int, int, int, int>, std::vector<int>> groups;
-  for (int i = 0; i < n_inst; i++)
-    groups[std::make_tuple(r->inst_C[i], specs[i].pass.n, r->inst_n1[i], specs[i].pass.method)]
-        .push_back(i);
-  long long want = 0;
-  for (auto& g : groups) want += (long long)std::get<0>(g.first) * (long long)g.second.size();
-  std::vector<std::vector<int>> cl_members;
+  // ---- clusters: equal shares unless uneven ones promise a 5 % shorter launch ----
+  BatchPlan plan = plan_equal(n_inst, specs, r->inst_C, r->inst_n1, slots, f64, wave_runs());
+  for (bool wave : {false, true}) {
+    BatchPlan uneven;
+    if (given || !plan_uneven(n_inst, specs, r->inst_n1, ctx->info.cus, r->csz, ctx->info.lds_max,
+                              wave, &uneven) ||
+        uneven.span > 0.95 * plan.span)
+      continue;
+    r->inst_C = uneven.C;
+    if (geometry() == OFX_OK && wave_runs() == wave) plan = uneven;
+    r->inst_C = plan.C;
+  }
+  st = geometry();
+  if (st) {
+    delete r;
+    return st;
+  }
+  const std::vector<std::vector<int>>& cl_members = plan.members;
   std::vector<int> cl_C, cl_method;
-  for (auto& g : groups) {
-    const int C = std::get<0>(g.first);
-    std::vector<int> ids = g.second;
-    long long ncl = (long long)ids.size();
-    if (want > slots) ncl = std::max(1LL, (long long)ids.size() * slots / want);
-    ncl = std::min(ncl, (long long)std::max(1, slots / C));
-    std::sort(ids.begin(), ids.end(), [&](int a, int b) {
-      const double ca = (double)specs[a].pass.nsteps, cb = (double)specs[b].pass.nsteps;
-      return ca != cb ? ca > cb : a < b;
-    });
-    std::vector<std::vector<int>> mem((size_t)ncl);
-    std::vector<double> load((size_t)ncl, 0.0);
-    for (int id : ids) {
-      size_t best = 0;
-      for (size_t c = 1; c < load.size(); c++)
-        if (load[c] < load[best]) best = c;
-      mem[best].push_back(id);
-      load[best] += (double)specs[id].pass.nsteps;
-    }
-    for (auto& m : mem) {
-      if (m.empty()) continue;
-      cl_members.push_back(m);
-      cl_C.push_back(C);
-      cl_method.push_back(std::get<3>(g.first));
-    }
+  for (const auto& m : cl_members) {
+    cl_C.push_back(r->inst_C[m[0]]);
+    cl_method.push_back(specs[m[0]].pass.method);
   }
   long long used = 0;
   for (int C : cl_C) used += C;
