@@ -24,7 +24,7 @@ HIP_FLAGS = [
 ]
 
 LIB_SOURCES = ["ofx_backend_hip.hip", "ofx_backend_rkl.hip", "ofx_backend_wave.hip",
-               "ofx_backend_wave_fixed.hip", "ofx_runtime.cpp", "ofx_mlp.hip", "ofx_qpm.hip",
+               "ofx_backend_wave_fixed.hip", "ofx_backend_wave_rk23.hip", "ofx_runtime.cpp", "ofx_mlp.hip", "ofx_qpm.hip",
                "ofx_gnlse.hip", "ofx_gnlse_wide.hip"]
 
 

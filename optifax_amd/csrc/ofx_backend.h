@@ -10,8 +10,8 @@
 // every instance of the launch is RK23 (ofx_backend_rkl.hip).
 enum { XMODE_RK23_LDS = 2 };
 // Bits 4..6: the wave kernel (ofx_wave_impl.h) with this many points a thread
-// (1, 2 or 4); bit 7: its form for workgroups of more than 256 threads.  The
-// other bits are then 0.  Bits 8..12 instead: the wave kernel with the default
+// (1, 2 or 4); bit 7: its form for workgroups of more than 256 threads.  Bit 1
+// is then its RK23 form (ofx_wave_rk23.h), bit 0 has no meaning.  Bits 8..12 instead: the wave kernel with the default
 // geometry of a grid of 2^that many points fixed.
 enum {
   XMODE_WAVE_SHIFT = 4,

@@ -30,17 +30,22 @@ const void* rkl_kernel(int precision, int xmode);
 const void* wave_kernel_fn(int precision, int points, bool wide);
 // the same with a grid size's default geometry fixed (ofx_backend_wave_fixed.hip)
 const void* wave_fixed_fn(int precision, int lg);
+// the RK23 forms of both (ofx_backend_wave_rk23.hip)
+const void* wave_rk23_fn(int precision, int points, bool wide);
+const void* wave_rk23_fixed_fn(int precision, int lg);
 
 // the kernel instantiation for a precision and xmode (exchange mode in bit 0,
 // XMODE_RK23_LDS in bit 1, the wave kernel's points a thread in bits 4..6, its
 // fixed grid size in bits 8..12)
 static const void* pass_fn(int precision, int xmode) {
+  const bool rk23 = (xmode & XMODE_RK23_LDS) != 0;
   if (xmode & XMODE_FIXED_MASK)
-    return wave_fixed_fn(precision, (xmode & XMODE_FIXED_MASK) >> XMODE_FIXED_SHIFT);
+    return (rk23 ? wave_rk23_fixed_fn : wave_fixed_fn)(
+        precision, (xmode & XMODE_FIXED_MASK) >> XMODE_FIXED_SHIFT);
   if (xmode & XMODE_WAVE_MASK)
-    return wave_kernel_fn(precision, (xmode & XMODE_WAVE_MASK) >> XMODE_WAVE_SHIFT,
-                          (xmode & XMODE_WAVE_WIDE) != 0);
-  if (xmode & XMODE_RK23_LDS) return rkl_kernel(precision, xmode & 1);
+    return (rk23 ? wave_rk23_fn : wave_kernel_fn)(
+        precision, (xmode & XMODE_WAVE_MASK) >> XMODE_WAVE_SHIFT, (xmode & XMODE_WAVE_WIDE) != 0);
+  if (rk23) return rkl_kernel(precision, xmode & 1);
   xmode &= 1;
   if (precision == OFX_F64)
     return xmode == XM_BARRIER ? (const void*)pass_kernel<double, XM_BARRIER>
@@ -153,16 +158,21 @@ int be_create(int device, Backend** out, DeviceInfo* info) {
     const int dyn = info->lds_max - 1024;
     bool ok = true;
     for (int prec : {OFX_F32, OFX_F64})
-      for (int xm : {XM_TAGS, XM_BARRIER, XM_TAGS | XMODE_RK23_LDS, XM_BARRIER | XMODE_RK23_LDS,
-                     1 << XMODE_WAVE_SHIFT, 2 << XMODE_WAVE_SHIFT, 4 << XMODE_WAVE_SHIFT,
-                     1 << XMODE_WAVE_SHIFT | XMODE_WAVE_WIDE, 2 << XMODE_WAVE_SHIFT | XMODE_WAVE_WIDE,
-                     4 << XMODE_WAVE_SHIFT | XMODE_WAVE_WIDE})
+      for (int xm : {XM_TAGS, XM_BARRIER, XM_TAGS | XMODE_RK23_LDS, XM_BARRIER | XMODE_RK23_LDS})
         ok = ok && hipFuncSetAttribute(pass_fn(prec, xm), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        dyn) == hipSuccess;
     for (int prec : {OFX_F32, OFX_F64})
+      for (int xm : {1 << XMODE_WAVE_SHIFT, 2 << XMODE_WAVE_SHIFT, 4 << XMODE_WAVE_SHIFT,
+                     1 << XMODE_WAVE_SHIFT | XMODE_WAVE_WIDE, 2 << XMODE_WAVE_SHIFT | XMODE_WAVE_WIDE,
+                     4 << XMODE_WAVE_SHIFT | XMODE_WAVE_WIDE})
+        for (int rk23 : {0, (int)XMODE_RK23_LDS})
+          ok = ok && hipFuncSetAttribute(pass_fn(prec, xm | rk23),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, dyn) == hipSuccess;
+    for (int prec : {OFX_F32, OFX_F64})
       for (int lg = WAVE_FIXED_LG; lg <= 16; lg++)
-        ok = ok && hipFuncSetAttribute(pass_fn(prec, lg << XMODE_FIXED_SHIFT),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, dyn) == hipSuccess;
+        for (int rk23 : {0, (int)XMODE_RK23_LDS})
+          ok = ok && hipFuncSetAttribute(pass_fn(prec, lg << XMODE_FIXED_SHIFT | rk23),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, dyn) == hipSuccess;
     if (!ok)
       snprintf(info->name + strlen(info->name), sizeof info->name - strlen(info->name),
                " [dyn-LDS attribute not set]");

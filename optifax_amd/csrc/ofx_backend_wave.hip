@@ -18,7 +18,7 @@ __global__ void __launch_bounds__(MAXT) wave_kernel(LaunchArgs a) {
   __shared__ double red[64];
   __shared__ int sflag[4];
   WvThread<R, S> thr;
-  wave_main<R, S, WvGeoRt, sizeof(R) == 8 || (MAXT > 256)>(
+  wave_main<R, S, WvGeoRt<>, sizeof(R) == 8 || (MAXT > 256)>(
       a, (int)blockIdx.x, reinterpret_cast<cpx<R>*>(ofx_lds_raw), red, sflag, &thr);
 }
 

@@ -10,7 +10,7 @@ namespace ofx {
 
 template <typename R, int LG>
 struct FixedGeometry {
-  static constexpr WaveGeometry g = wave_geometry(LG, sizeof(R) == 8);
+  static constexpr WaveGeometry g = wave_geometry(LG, sizeof(R) == 8, false);
   static constexpr int share = (1 << LG) >> g.lgC, S = share > g.block ? share / g.block : 1;
   typedef WvGeoCt<LG, g.lgC, g.block> Geo;
 };

@@ -39,11 +39,27 @@ enum {
 // Threads: 4 transform elements each where that leaves the stages at most 2
 // points a thread (2^12 FP32 at 16 workgroups: 128 threads 6.3, 256 5.3; 2^15
 // at 128: 128 threads 9.9, 256 8.0, 512 10.2).
+// RK23 (a member owns 4 columns or more; FP64 2^16 does not fit LDS):
+//   2^8   1: 2.9 / 3.4, 2: 6.2 / 7.8                      : 8.1 / 9.5
+//   2^9   1: 3.5 / 4.3, 4: 6.5 / 8.1                      : 8.8 / 10.5
+//   2^10  1: 4.5 / 6.4, 4: 6.2 / 7.8, 8: 7.0 / 8.9        : 9.5 / 11.0
+//   2^11  8: 5.8 / 8.1, 16: 7.2 / 10.2                    : 10.0 / 11.7
+//   2^12  8: 8.4 / 11.1, 16: 6.7 / 8.3                    : 11.4 / 13.1
+//   2^13  16: 8.1 / 12.0, 32: 6.8 / 10.0                  : 11.3 / 14.7
+//   2^14  16: 11.8 / -, 32: 10.0 / 17.1                   : 16.1 / 20.0
+//   2^15  32: 14.9 / -, 64: 9.3 / 16.7                    : 18.1 / 22.4
+//   2^16  64: 13.4 / -                                    : 23.6 / -
+// (FP32 2^14 at 32 workgroups: 256 threads 11.7, 512 10.0; FP64's 512-thread
+// form spills.)
 enum { WAVE_FIXED_LG = 8 };
 struct WaveGeometry {
   int lgC, block;
 };
-constexpr WaveGeometry wave_geometry(int lg, bool f64) {
+constexpr WaveGeometry wave_geometry(int lg, bool f64, bool rk23) {
+  if (rk23)
+    return lg <= 10   ? WaveGeometry{0, lg < 6 ? 64 : lg < 8 ? 1 << lg : 256}
+           : lg <= 13 ? WaveGeometry{lg == 11 ? 3 : lg - 8, 256}
+                      : WaveGeometry{lg == 14 ? 5 : 6, f64 ? 256 : 512};
   return lg <= 10   ? WaveGeometry{0, lg < 6 ? 64 : lg < 8 ? 1 << lg : lg < 10 || f64 ? 256 : 512}
          : lg == 11 ? WaveGeometry{4, 128}
          : lg == 12 ? WaveGeometry{4, 256}

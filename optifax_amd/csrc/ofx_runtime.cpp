@@ -135,21 +135,23 @@ int max_cluster(int method, int n1, int n2) {
   return method == OFX_METHOD_RK23 ? std::min(n1 / 4, n2) : std::min(n1, n2);
 }
 
-// LDS of a workgroup of the wave kernel: A0 with its halo, the column slots
-// (272 elements each 256) and the row slots (ofx_wave_impl.h)
-size_t wave_lds_bytes(int n1, int n2, int C, size_t csz) {
-  const size_t W = n1 / C, Rr = n2 / C, LC = W + 4;
-  return (LC * (size_t)(n2 + 1) +
+// LDS of a workgroup of the wave kernel: A0 with its halo (RK23: and two K1 of
+// the same layout), the column slots (272 elements each 256) and the row slots
+// (ofx_wave_impl.h)
+size_t wave_lds_bytes(int n1, int n2, int C, int method, size_t csz) {
+  const bool rk23 = method == OFX_METHOD_RK23;
+  const size_t W = n1 / C, Rr = n2 / C, LC = W + 2 * halo_of(method);
+  return ((rk23 ? 3 : 1) * LC * (size_t)(n2 + 1) +
           ((LC * n2 + 255) / 256 + (Rr * n1 + 255) / 256) * 272) * csz;
 }
 
 // Points a thread with which the wave kernel can run an instance (1, 2 or 4),
-// or 0 when it cannot: Heun, transforms of at most 256, at most 4 points a
+// or 0 when it cannot: transforms of at most 256, at most 4 points a
 // thread, every column row with a thread, at most two error records a lane.
 int wave_points(const ofx_pass_params& p, int n1, int C, int block, size_t csz, int lds_max) {
   const int n2 = p.n / n1, share = p.n / C;
-  if (p.method != OFX_METHOD_HEUN || n1 > 256 || n2 > 256 || C > 128 || ilog2i(block) < 0 ||
-      block < n2 || share > 4 * block || (int)wave_lds_bytes(n1, n2, C, csz) > lds_max - 1024)
+  if (n1 > 256 || n2 > 256 || C > 128 || ilog2i(block) < 0 || block < n2 || share > 4 * block ||
+      (int)wave_lds_bytes(n1, n2, C, p.method, csz) > lds_max - 1024)
     return 0;
   return share > 2 * block ? 4 : share > block ? 2 : 1;
 }
@@ -162,8 +164,8 @@ int wave_points(const ofx_pass_params& p, int n1, int C, int block, size_t csz, 
 // kernel's 16.5).
 int wave_cluster(const ofx_pass_params& p, int n1, int n_inst, int cus, size_t csz) {
   const int n = p.n;
-  if (p.method != OFX_METHOD_HEUN || n1 > 256 || n / n1 > 256) return 0;
-  int C = 1 << wave_geometry(ilog2i(n), csz == 16).lgC;
+  if (n1 > 256 || n / n1 > 256) return 0;
+  int C = 1 << wave_geometry(ilog2i(n), csz == 16, p.method == OFX_METHOD_RK23).lgC;
   while (C > 1 && (long long)n_inst * C > cus) C >>= 1;
   const bool fits = n / C <= 1024 && (long long)n_inst * C <= cus;
   return fits && C <= max_cluster(p.method, n1, n / n1) ? C : 0;
@@ -274,9 +276,11 @@ int check_pass(ofx_context* ctx, const ofx_pass_params* p) {
 }
 
 // Launch geometry of one instance of a batch of n_inst: the four-step split
-// n1 (N = n1 n2) and the cluster size C (workgroups per instance).
+// n1 (N = n1 n2) and the cluster size C (workgroups per instance).  waves: the
+// wave kernel may run it.
 int plan_instance(ofx_context* ctx, const ofx_pass_params& p, int n_inst, const ofx_tuning* tune,
-                  int spec_cluster, int spec_n1, size_t csz, int* C_out, int* n1_out) {
+                  int spec_cluster, int spec_n1, size_t csz, bool waves, int* C_out,
+                  int* n1_out) {
   const int n = p.n, lg = ilog2i(n);
   int n1 = 1 << ((lg + 1) / 2);
   if (tune && tune->n1) n1 = tune->n1;
@@ -304,7 +308,7 @@ int plan_instance(ofx_context* ctx, const ofx_pass_params& p, int n_inst, const 
         (int)lds_bytes_for(n1, n2, C, meth, csz) > ctx->info.lds_max - 1024)
       return fail(ctx, OFX_E_ARG, "cluster size %d is invalid for N=%d (n1=%d)", C, n, n1);
   } else if (const int Cw = tune && tune->exchange == 2 ? 0
-                            : wave_cluster(p, n1, n_inst, ctx->info.cus, csz)) {
+                            : waves ? wave_cluster(p, n1, n_inst, ctx->info.cus, csz) : 0) {
     C = Cw;
   } else {
     // The general kernel: spread a small batch over more workgroups until a
@@ -329,8 +333,8 @@ int plan_instance(ofx_context* ctx, const ofx_pass_params& p, int n_inst, const 
 // FP64 fields (whose 512-thread form spills: 26 against 17.3).  0 when the wave
 // kernel cannot run the instance.
 int wave_block(const ofx_pass_params& p, int n1, int C, size_t csz, int lds_max) {
-  const int n2 = p.n / n1, el = C == 1 ? p.n : (n1 / C + 4) * n2;
-  const WaveGeometry g = wave_geometry(ilog2i(p.n), csz == 16);
+  const int n2 = p.n / n1, el = C == 1 ? p.n : (n1 / C + 2 * halo_of(p.method)) * n2;
+  const WaveGeometry g = wave_geometry(ilog2i(p.n), csz == 16, p.method == OFX_METHOD_RK23);
   int block = 64;
   while (block < el / 4 || block < n2 || (C == 1 && block < std::min(p.n, 256))) block <<= 1;
   block = C == 1 << g.lgC ? g.block : std::min(block, csz == 8 ? 512 : 256);
@@ -342,8 +346,8 @@ int wave_block(const ofx_pass_params& p, int n1, int C, size_t csz, int lds_max)
 // instance (2^8 2.6 against 4.1 us per step, 2^12 5.8 against 7.3, 2^15 8.1
 // against 9.2; FP64 2^15 11.0 against 13.4), else the one for any geometry.
 // lg: log2 of the common grid size of the instances, or 0.
-int wave_mode(int points, int block, int lg, int n1, int C, size_t csz) {
-  const WaveGeometry g = wave_geometry(lg, csz == 16);
+int wave_mode(int points, int block, int lg, int n1, int C, int method, size_t csz) {
+  const WaveGeometry g = wave_geometry(lg, csz == 16, method == OFX_METHOD_RK23);
   if (lg >= WAVE_FIXED_LG && n1 == 1 << ((lg + 1) / 2) && C == 1 << g.lgC && block == g.block)
     return lg << XMODE_FIXED_SHIFT;
   return (points << XMODE_WAVE_SHIFT) | (block > 256 ? XMODE_WAVE_WIDE : 0);
@@ -379,10 +383,13 @@ int exchange_mode(int exchange, int cmin) {
 // 14.6 at 1024, FP64 2^12 13.2 and 2^15 20.6.  Only ratios are used.
 double step_us(const ofx_pass_params& p, int C, bool f64, bool wave) {
   const double x = ilog2i(p.n) - 14, share = (double)p.n / C;
-  if (wave) return f64 ? 13.6 + 1.3 * x + 4.5e-3 * share : 6.9 + 0.7 * x + 6.5e-3 * share;
+  const bool rk23 = p.method == OFX_METHOD_RK23;
+  if (wave)
+    return (rk23 ? 1.35 : 1.0) *
+           (f64 ? 13.6 + 1.3 * x + 4.5e-3 * share : 6.9 + 0.7 * x + 6.5e-3 * share);
   const double t = f64 ? 13.0 + 1.2 * x + 9.2e-3 * share
                        : 12.5 + 1.2 * x + 5.2e-3 * share + 1.7e-3 * std::max(0.0, share - 2048);
-  return p.method == OFX_METHOD_RK23 ? 1.2 * std::max(t, 4.0) : std::max(t, 4.0);
+  return rk23 ? 1.2 * std::max(t, 4.0) : std::max(t, 4.0);
 }
 
 // Instances to clusters: a cluster runs its members one after the other.
@@ -452,7 +459,8 @@ bool plan_uneven(int n_inst, const ofx_opo_spec* specs, const std::vector<int>& 
   for (int i = 0; i < n_inst; i++) {
     const ofx_pass_params& p = specs[i].pass;
     const int n1 = inst_n1[i], n2 = p.n / n1;
-    const int top = wave ? 1 << wave_geometry(ilog2i(p.n), f64).lgC : 128;
+    const int top =
+        wave ? 1 << wave_geometry(ilog2i(p.n), f64, p.method == OFX_METHOD_RK23).lgC : 128;
     for (int C = 1; C <= std::min(std::min(max_cluster(p.method, n1, n2), top), cus); C <<= 1) {
       if (wave ? !wave_block(p, n1, C, csz, lds_max)
                : ((int)lds_bytes_for(n1, n2, C, p.method, csz) > lds_max - 1024 ||
@@ -581,10 +589,15 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
   r->inst_C.resize(n_inst);
   r->inst_n1.resize(n_inst);
   int nmax = 0;
+  bool all_rk23 = n_inst > 0;
+  for (int i = 0; i < n_inst; i++)
+    all_rk23 = all_rk23 && specs[i].pass.method == OFX_METHOD_RK23;
+  // (a launch runs one kernel: RK23 beside Heun is the general one's)
+  auto waves = [&](int i) { return all_rk23 || specs[i].pass.method == OFX_METHOD_HEUN; };
   for (int i = 0; i < n_inst; i++) {
     nmax = std::max(nmax, specs[i].pass.n);
     st = plan_instance(ctx, specs[i].pass, n_inst, tune, specs[i].cluster, specs[i].n1, r->csz,
-                       &r->inst_C[i], &r->inst_n1[i]);
+                       waves(i), &r->inst_C[i], &r->inst_n1[i]);
     if (st) {
       delete r;
       return st;
@@ -593,18 +606,16 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
   r->nmax = nmax;
   const int exchange = tune ? tune->exchange : 0;
   bool given = n_inst < 2 || (tune && (tune->cluster || tune->block || tune->exchange));
-  bool all_rk23 = n_inst > 0;
-  for (int i = 0; i < n_inst; i++) {
-    given = given || specs[i].cluster;
-    all_rk23 = all_rk23 && specs[i].pass.method == OFX_METHOD_RK23;
-  }
+  for (int i = 0; i < n_inst; i++) given = given || specs[i].cluster;
   // threads, launch mode and LDS for the cluster sizes in r->inst_C
   int slots = 0;
   auto geometry = [&]() -> int {
     int cmin = 1 << 30, wblock = 0;
     for (int i = 0; i < n_inst; i++) {
       cmin = std::min(cmin, r->inst_C[i]);
-      const int b = wave_block(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->csz, ctx->info.lds_max);
+      const int b = waves(i) ? wave_block(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->csz,
+                                          ctx->info.lds_max)
+                             : 0;
       wblock = i && !wblock ? 0 : b ? std::max(wblock, b) : 0;
     }
     if (int st = plan_block(ctx, tune, cmin, wblock, &r->block)) return st;
@@ -612,8 +623,9 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
     // tagged exchange has it wherever it can run)
     int points = 0;
     for (int i = 0; i < n_inst && (exchange == 1 || (exchange == 0 && wblock)); i++) {
-      const int w = wave_points(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->block, r->csz,
-                                ctx->info.lds_max);
+      const int w = waves(i) ? wave_points(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->block,
+                                           r->csz, ctx->info.lds_max)
+                             : 0;
       points = w ? std::max(points, w) : 0;
       if (!w) break;
     }
@@ -622,11 +634,12 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
     for (int i = 0; i < n_inst; i++) {
       const int n = specs[i].pass.n, n1 = r->inst_n1[i], C = r->inst_C[i];
       same = same && n == specs[0].pass.n && n1 == r->inst_n1[0] && C == r->inst_C[0];
-      r->lds = std::max(r->lds, points ? wave_lds_bytes(n1, n / n1, C, r->csz)
-                                       : lds_bytes_for(n1, n / n1, C, specs[i].pass.method, r->csz));
+      const int method = specs[i].pass.method;
+      r->lds = std::max(r->lds, points ? wave_lds_bytes(n1, n / n1, C, method, r->csz)
+                                       : lds_bytes_for(n1, n / n1, C, method, r->csz));
     }
     r->xmode = points ? wave_mode(points, r->block, same ? ilog2i(specs[0].pass.n) : 0, r->inst_n1[0],
-                                  r->inst_C[0], r->csz)
+                                  r->inst_C[0], specs[0].pass.method, r->csz)
                       : exchange_mode(exchange, cmin);
     if (all_rk23) r->xmode |= XMODE_RK23_LDS;
     const int bpc = be_blocks_per_cu(ctx->be, precision, r->xmode, r->block, r->lds);
@@ -1369,14 +1382,16 @@ extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params*
   // geometry: as ofx_opo_create plans a batch of equal instances (one
   // cluster per instance, all resident at once)
   int C = 0, n1 = 0, block = 0;
-  st = plan_instance(ctx, *p, batch, nullptr, 0, 0, 8, &C, &n1);
+  st = plan_instance(ctx, *p, batch, nullptr, 0, 0, 8, true, &C, &n1);
   const int wblock = st ? 0 : wave_block(*p, n1, C, 8, ctx->info.lds_max);
   if (!st) st = plan_block(ctx, nullptr, C, wblock, &block);
   if (st) return st;
   const int n2 = n / n1;
   const int points = wblock ? wave_points(*p, n1, C, block, 8, ctx->info.lds_max) : 0;
-  const int xmode = points ? wave_mode(points, block, ilog2i(n), n1, C, 8) : exchange_mode(0, C);
-  const size_t lds = points ? wave_lds_bytes(n1, n2, C, 8) : lds_bytes_for(n1, n2, C, method, 8);
+  const int xmode = points ? wave_mode(points, block, ilog2i(n), n1, C, method, 8) |
+                                 (method == OFX_METHOD_RK23 ? (int)XMODE_RK23_LDS : 0)
+                           : exchange_mode(0, C);
+  const size_t lds = points ? wave_lds_bytes(n1, n2, C, method, 8) : lds_bytes_for(n1, n2, C, method, 8);
   const int bpc = be_blocks_per_cu(ctx->be, OFX_F32, xmode, block, lds);
   if (bpc < 1)
     return fail(ctx, OFX_E_ARG, "kernel cannot launch with block=%d and %zu bytes of LDS", block, lds);

@@ -1,5 +1,5 @@
-// Body of the wave kernel: the adaptive Heun pass and the round trip of
-// ofx_pass_impl.h for clusters whose members hold a small share of the field
+// Body of the wave kernel: the adaptive Heun pass (RK23: ofx_wave_rk23.h) and the
+// round trip of ofx_pass_impl.h for clusters whose members hold a small share of the field
 // (at most 4 points a thread), where a step is a chain of latencies.
 //
 // The decomposition, the exchange buffers, the tags and the arithmetic of
@@ -110,11 +110,11 @@ OFX_DEV cpx<R> wv_rounded(cpx<R> v) {
 
 // State of one thread.  On the device one object per thread, in registers; in
 // the emulation an array that each phase walks.
-template <typename R, int S>
+template <typename R, int S, int HW = 2>
 struct WvThread {
   typedef cpx<R> C;
   C v[4];                  // transform elements j + m L/4
-  C wt[S + 4];             // exp(i w0 t) of the stage window
+  C wt[S + 2 * HW];        // exp(i w0 t) of the stage window
   C twr[3][3], twc[3][3];  // twiddles of the passes after each exchange (rows, columns)
   C fc[4], fr[4];          // four-step factors of the own column / row elements
   C ph[4];                 // dispersion phasors for the step length held
@@ -244,9 +244,12 @@ OFX_DEV double wv_wave_max(double v) {
 }
 #endif
 
-// Launch geometry of a member: read from the instance and the launch ...
+// Launch geometry of a member (HW: halo columns on each side): read from the
+// instance and the launch ...
+template <int HW_ = 2>
 struct WvGeoRt {
   static constexpr bool FIXED = false;
+  static constexpr int HW = HW_;
   int n, n1, n2, lg1, lg2, lgW, Cn, W, Rr, LC, sT, NT, nw;
   OFX_DEV void set(const InstDesc& d, int C, int block) {
     n = d.n;
@@ -260,7 +263,7 @@ struct WvGeoRt {
     W = n1 >> lgC;
     lgW = lg1 - lgC;
     Rr = n2 >> lgC;
-    LC = W + 4;
+    LC = W + 2 * HW;
     sT = n2 + 1;
     NT = block;
     nw = NT >> 6;
@@ -269,12 +272,12 @@ struct WvGeoRt {
 // ... or fixed for a grid size's default geometry: shifts, strides, slot and
 // wave counts are then constants (about half of a step's instructions form
 // indices otherwise).
-template <int LG, int LGC, int NT_>
+template <int LG, int LGC, int NT_, int HW_ = 2>
 struct WvGeoCt {
   static constexpr bool FIXED = true;
   static constexpr int n = 1 << LG, lg1 = (LG + 1) / 2, lg2 = LG - lg1, n1 = 1 << lg1, n2 = 1 << lg2,
-                       Cn = 1 << LGC, W = n1 >> LGC, lgW = lg1 - LGC, Rr = n2 >> LGC, LC = W + 4,
-                       sT = n2 + 1, NT = NT_, nw = NT >> 6;
+                       Cn = 1 << LGC, W = n1 >> LGC, lgW = lg1 - LGC, Rr = n2 >> LGC, HW = HW_,
+                       LC = W + 2 * HW, sT = n2 + 1, NT = NT_, nw = NT >> 6;
   OFX_DEV void set(const InstDesc&, int, int) {}
 };
 
@@ -283,10 +286,10 @@ template <typename R, int S, typename GEO, bool REFRESH>
 struct WvRun : GEO {
   typedef cpx<R> C;
   typedef Tagged<C> TT;
-  typedef WvThread<R, S> T;
+  typedef WvThread<R, S, GEO::HW> T;
   using GEO::n; using GEO::n1; using GEO::n2; using GEO::lg1; using GEO::lg2; using GEO::lgW;
   using GEO::Cn; using GEO::W; using GEO::Rr; using GEO::LC; using GEO::sT; using GEO::NT;
-  using GEO::nw;
+  using GEO::nw; using GEO::HW;
   const LaunchArgs& a;
   const ClusterDesc& cd;
   const InstDesc& d;
@@ -295,10 +298,9 @@ struct WvRun : GEO {
   int* sflag;    // [0] barrier verdict, [1] a poll gave up
   T* thr;
   int rank, wv, tid, c0, k20;
-  C *A0, *X, *Tb;
+  C *A0, *X, *Tb, *K1;   // (K1: RK23 only, two buffers of A0's layout)
   u64 *t1b, *t2b, *slots;
   int* abort_flag;
-  static constexpr int HW = 2;
 
   OFX_DEV WvRun(const LaunchArgs& a_, const ClusterDesc& cd_, const InstDesc& d_, SyncState& sy_,
                 double* red_, int* sflag_, T* thr_)
@@ -474,7 +476,7 @@ struct WvRun : GEO {
       }
       const int r = tid & (n2 - 1), s0 = (tid >> lg2) * S;
 #pragma unroll
-      for (int i = 0; i < S + 4; i++) {
+      for (int i = 0; i < S + 2 * HW; i++) {
         const int lc = s0 + i < LC ? s0 + i : LC - 1;
         const int j = (c0 - HW + lc + n1 * r) & (n - 1);
         t.wt[i] = wv_mulq(wtg[(j >> lg1) * n1], wtg[j & (n1 - 1)]);
@@ -680,6 +682,10 @@ struct WvRun : GEO {
     return !fail;
   }
 
+  // one adaptive RK23 pass (ofx_wave_rk23.h)
+  OFX_DEV int rk23(R cc, long long& att, long long& acc, double& s_held);
+  OFX_DEV bool boundary_in(unsigned x, unsigned tag, C* dst);
+
   OFX_DEV void run(int rank_, C* lds);
 };
 
@@ -704,6 +710,7 @@ OFX_DEV void WvRun<R, S, GEO, REFRESH>::run(int rank_, C* lds) {
   A0 = lds;
   X = A0 + LC * sT;
   Tb = X + ((LC * n2 + 255) >> 8) * WV_SLOT;
+  K1 = Tb + ((Rr * n1 + 255) >> 8) * WV_SLOT;
   C* field = (C*)d.field;
   const double dt = d.dt;
   const R cc = (R)(0.5 / dt / d.w0);
@@ -745,11 +752,17 @@ OFX_DEV void WvRun<R, S, GEO, REFRESH>::run(int rank_, C* lds) {
       each([&](int tid, int, T&) {
         for (int j = tid; j < nsteps; j += NT) gl(stepmods)[j] = 0.0f;
       });
+    if constexpr (HW == 4) {
+      status = rk23(cc, trip_att, trip_acc, s_held);
+      attempts += trip_att;
+      accepted += trip_acc;
+      chunk = (int)nChunks + 1;  // (no Heun loop)
+    }
     double Gk = (double)chunk <= nChunks ? uniform(gl(Gd)[(int)k - 1]) : 0.0;
     // exp(-i bdwz) at both ends of the step
     C eb0 = expi(-(bdiffw0 * (k - 1.0) * hmin), R(0));
     C eb1 = expi(-(bdiffw0 * (k - 1.0 + stepmod) * hmin), R(0));
-    while ((double)chunk <= nChunks) {
+    if constexpr (HW == 2) while ((double)chunk <= nChunks) {
       refresh();
       const R gk = (R)(hmin * stepmod * Gk);
       // ---- both stages, corrector, error quotient, absorber ----
@@ -1024,7 +1037,7 @@ OFX_DEV void WvRun<R, S, GEO, REFRESH>::run(int rank_, C* lds) {
 
 template <typename R, int S, typename GEO, bool REFRESH>
 OFX_DEV void wave_main(const LaunchArgs& a, int wg, cpx<R>* lds, double* red, int* sflag,
-                       WvThread<R, S>* thr) {
+                       WvThread<R, S, GEO::HW>* thr) {
   const int ci = a.wg_cluster[wg];
   if (ci < 0) return;
   const ClusterDesc& cd = a.clusters[ci];

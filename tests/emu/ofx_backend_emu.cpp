@@ -21,7 +21,7 @@
 #include "../../include/optifax_hip.h"
 #include "../../optifax_amd/csrc/ofx_backend.h"
 #include "../../optifax_amd/csrc/ofx_pass_impl.h"
-#include "../../optifax_amd/csrc/ofx_wave_impl.h"
+#include "../../optifax_amd/csrc/ofx_wave_rk23.h"
 
 namespace ofx {
 
@@ -92,43 +92,43 @@ static void run_wg(const LaunchArgs* a, int wg, size_t lds) {
 }
 
 // the wave kernel: a workgroup's threads are walked phase by phase
-template <typename R, int S>
+template <typename R, int S, int HW>
 static void run_wave(const LaunchArgs* a, int wg, size_t lds) {
   std::vector<unsigned char> mem(lds + 64);
-  std::vector<WvThread<R, S>> thr((size_t)a->block);
+  std::vector<WvThread<R, S, HW>> thr((size_t)a->block);
   double red[64];
   int sflag[4];
-  wave_main<R, S, WvGeoRt, false>(*a, wg, reinterpret_cast<cpx<R>*>(mem.data()), red, sflag, thr.data());
+  wave_main<R, S, WvGeoRt<HW>, false>(*a, wg, reinterpret_cast<cpx<R>*>(mem.data()), red, sflag, thr.data());
 }
-template <typename R>
+template <typename R, int HW>
 static void (*wave_fn(int points))(const LaunchArgs*, int, size_t) {
-  return points == 4 ? run_wave<R, 4> : points == 2 ? run_wave<R, 2> : run_wave<R, 1>;
+  return points == 4 ? run_wave<R, 4, HW> : points == 2 ? run_wave<R, 2, HW> : run_wave<R, 1, HW>;
 }
 
 // its forms with a fixed default geometry
-template <typename R, int LG>
+template <typename R, int HW, int LG>
 static void run_fixed(const LaunchArgs* a, int wg, size_t lds) {
-  constexpr WaveGeometry g = wave_geometry(LG, sizeof(R) == 8);
+  constexpr WaveGeometry g = wave_geometry(LG, sizeof(R) == 8, HW == 4);
   constexpr int share = (1 << LG) >> g.lgC, S = share > g.block ? share / g.block : 1;
   std::vector<unsigned char> mem(lds + 64);
-  std::vector<WvThread<R, S>> thr((size_t)a->block);
+  std::vector<WvThread<R, S, HW>> thr((size_t)a->block);
   double red[64];
   int sflag[4];
-  wave_main<R, S, WvGeoCt<LG, g.lgC, g.block>, false>(
+  wave_main<R, S, WvGeoCt<LG, g.lgC, g.block, HW>, false>(
       *a, wg, reinterpret_cast<cpx<R>*>(mem.data()), red, sflag, thr.data());
 }
-template <typename R>
+template <typename R, int HW>
 static void (*fixed_fn(int lg))(const LaunchArgs*, int, size_t) {
   switch (lg) {
-    case 8: return run_fixed<R, 8>;
-    case 9: return run_fixed<R, 9>;
-    case 10: return run_fixed<R, 10>;
-    case 11: return run_fixed<R, 11>;
-    case 12: return run_fixed<R, 12>;
-    case 13: return run_fixed<R, 13>;
-    case 14: return run_fixed<R, 14>;
-    case 15: return run_fixed<R, 15>;
-    default: return run_fixed<R, 16>;
+    case 8: return run_fixed<R, HW, 8>;
+    case 9: return run_fixed<R, HW, 9>;
+    case 10: return run_fixed<R, HW, 10>;
+    case 11: return run_fixed<R, HW, 11>;
+    case 12: return run_fixed<R, HW, 12>;
+    case 13: return run_fixed<R, HW, 13>;
+    case 14: return run_fixed<R, HW, 14>;
+    case 15: return run_fixed<R, HW, 15>;
+    default: return run_fixed<R, HW, 16>;
   }
 }
 
@@ -149,10 +149,16 @@ int be_launch(Backend* b, const LaunchArgs& a, int precision, int xmode, int gri
     for (int wg = 0; wg < grid; wg++) {
       if (xmode & XMODE_FIXED_MASK) {
         const int lg = (xmode & XMODE_FIXED_MASK) >> XMODE_FIXED_SHIFT;
-        th.emplace_back(precision == OFX_F64 ? fixed_fn<double>(lg) : fixed_fn<float>(lg), &a, wg, lds);
+        th.emplace_back(xmode & XMODE_RK23_LDS
+                            ? (precision == OFX_F64 ? fixed_fn<double, 4>(lg) : fixed_fn<float, 4>(lg))
+                            : (precision == OFX_F64 ? fixed_fn<double, 2>(lg) : fixed_fn<float, 2>(lg)),
+                        &a, wg, lds);
       } else if (xmode & XMODE_WAVE_MASK) {
         const int pts = (xmode & XMODE_WAVE_MASK) >> XMODE_WAVE_SHIFT;
-        th.emplace_back(precision == OFX_F64 ? wave_fn<double>(pts) : wave_fn<float>(pts), &a, wg, lds);
+        th.emplace_back(xmode & XMODE_RK23_LDS
+                            ? (precision == OFX_F64 ? wave_fn<double, 4>(pts) : wave_fn<float, 4>(pts))
+                            : (precision == OFX_F64 ? wave_fn<double, 2>(pts) : wave_fn<float, 2>(pts)),
+                        &a, wg, lds);
       } else if (xmode & XMODE_RK23_LDS)
         th.emplace_back(emu_rkl_fn(precision, xmode & 1), &a, wg, lds);
       else if (precision == OFX_F64)
