@@ -23,7 +23,7 @@ HIP_FLAGS = [
     "-Wno-unused-result", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
-LIB_SOURCES = ["ofx_backend_hip.hip", "ofx_backend_rkl.hip", "ofx_backend_wave.hip",
+LIB_SOURCES = ["ofx_backend_hip.hip", "ofx_backend_rkl.hip", "ofx_backend_sized.hip", "ofx_backend_wave.hip",
                "ofx_backend_wave_fixed.hip", "ofx_backend_wave_rk23.hip", "ofx_runtime.cpp", "ofx_mlp.hip", "ofx_qpm.hip",
                "ofx_gnlse.hip", "ofx_gnlse_wide.hip"]
 

@@ -9,6 +9,10 @@
 // whose RK23 pass reads the cluster descriptor from a copy in LDS, used when
 // every instance of the launch is RK23 (ofx_backend_rkl.hip).
 enum { XMODE_RK23_LDS = 2 };
+// Bit 2: the general kernel's form for Heun instances at a counter barrier in
+// workgroups of 512 threads, with the usual grid splits fixed at compile time
+// (ofx_backend_sized.hip).
+enum { XMODE_SIZED = 4, XMODE_SIZED_BLOCK = 512 };
 // Bits 4..6: the wave kernel (ofx_wave_impl.h) with this many points a thread
 // (1, 2 or 4); bit 7: its form for workgroups of more than 256 threads.  Bit 1
 // is then its RK23 form (ofx_wave_rk23.h), bit 0 has no meaning.  Bits 8..12 instead: the wave kernel with the default

@@ -26,6 +26,8 @@ __global__ void __launch_bounds__(512) pass_kernel(LaunchArgs a) {
 
 // the RK23 variant's kernels (ofx_backend_rkl.hip)
 const void* rkl_kernel(int precision, int xmode);
+// the general kernel with fixed grid splits (ofx_backend_sized.hip)
+const void* sized_kernel(int precision);
 // the wave kernels (ofx_backend_wave.hip)
 const void* wave_kernel_fn(int precision, int points, bool wide);
 // the same with a grid size's default geometry fixed (ofx_backend_wave_fixed.hip)
@@ -45,6 +47,7 @@ static const void* pass_fn(int precision, int xmode) {
   if (xmode & XMODE_WAVE_MASK)
     return (rk23 ? wave_rk23_fn : wave_kernel_fn)(
         precision, (xmode & XMODE_WAVE_MASK) >> XMODE_WAVE_SHIFT, (xmode & XMODE_WAVE_WIDE) != 0);
+  if (xmode & XMODE_SIZED) return sized_kernel(precision);
   if (rk23) return rkl_kernel(precision, xmode & 1);
   xmode &= 1;
   if (precision == OFX_F64)
@@ -158,7 +161,8 @@ int be_create(int device, Backend** out, DeviceInfo* info) {
     const int dyn = info->lds_max - 1024;
     bool ok = true;
     for (int prec : {OFX_F32, OFX_F64})
-      for (int xm : {XM_TAGS, XM_BARRIER, XM_TAGS | XMODE_RK23_LDS, XM_BARRIER | XMODE_RK23_LDS})
+      for (int xm : {XM_TAGS, XM_BARRIER, XM_TAGS | XMODE_RK23_LDS, XM_BARRIER | XMODE_RK23_LDS,
+                     XM_BARRIER | XMODE_SIZED})
         ok = ok && hipFuncSetAttribute(pass_fn(prec, xm), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        dyn) == hipSuccess;
     for (int prec : {OFX_F32, OFX_F64})

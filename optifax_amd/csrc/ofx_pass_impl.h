@@ -43,7 +43,9 @@ unsigned long long emu_clock();  // wall clock in the device's ticks
 #else
 #define OFX_DEV __device__ __forceinline__
 #define OFX_TID ((int)threadIdx.x)
+#ifndef OFX_NT   // (a translation unit may fix the workgroup's size)
 #define OFX_NT ((int)blockDim.x)
+#endif
 #define OFX_SYNC() __syncthreads()
 #endif
 
@@ -205,6 +207,75 @@ OFX_DEV cpx<R> k_term(cpx<R> nl, cpx<R> up, cpx<R> dn, R g, R cc) {
   return mkc<R>(g * iy, -g * ix);
 }
 
+// Products with their fused forms written out: left to the compiler, which of
+// a sum's two products is rounded first depends on the code around it, and
+// these are the forms that the general kernel's code has (so that kernels built
+// with them give the same bits).
+template <typename R>
+OFX_DEV R wv_fma(R a, R b, R c) {
+#ifdef OFX_EMU
+  return a * b + c;   // (the emulation's host code fuses nothing)
+#else
+  if constexpr (sizeof(R) == 4)
+    return __builtin_fmaf(a, b, c);
+  else
+    return __builtin_fma(a, b, c);
+#endif
+}
+// a b, the imaginary part's a.y b.x rounded first (FP64: the other one)
+template <typename R>
+OFX_DEV cpx<R> wv_mul(cpx<R> a, cpx<R> b) {
+  if constexpr (sizeof(R) == 8)
+    return mkc<R>(wv_fma(a.x, b.x, -(a.y * b.y)), wv_fma(a.y, b.x, a.x * b.y));
+  return mkc<R>(wv_fma(a.x, b.x, -(a.y * b.y)), wv_fma(a.x, b.y, a.y * b.x));
+}
+// a b, the imaginary part's a.x b.y rounded first
+template <typename R>
+OFX_DEV cpx<R> wv_mulq(cpx<R> a, cpx<R> b) {
+  return mkc<R>(wv_fma(a.x, b.x, -(a.y * b.y)), wv_fma(a.y, b.x, a.x * b.y));
+}
+// a conj(b)
+template <typename R>
+OFX_DEV cpx<R> wv_mulc(cpx<R> a, cpx<R> b) {
+  return mkc<R>(wv_fma(a.x, b.x, a.y * b.y), wv_fma(a.y, b.x, -(a.x * b.y)));
+}
+// |a|^2 in FP64
+template <typename R>
+OFX_DEV double wv_abs2(cpx<R> a) {
+  const double x = a.x, y = a.y;
+  return wv_fma(x, x, y * y);
+}
+// nl_term_e
+template <typename R>
+OFX_DEV cpx<R> wv_nl(cpx<R> A, cpx<R> e) {
+  const R yy = A.y * A.y;
+  const R a2 = R(2) * wv_fma(A.x, A.x, yy), sx = wv_fma(A.x, A.x, -yy), sy = R(2) * A.x * A.y;
+  const R im = sizeof(R) == 8 ? wv_fma(sy, e.x, sx * e.y) : wv_fma(sx, e.y, sy * e.x);
+  return mkc<R>(wv_fma(a2, e.x, wv_fma(sx, e.x, -(sy * e.y))), wv_fma(-a2, e.y, im));
+}
+
+// A product that is rounded before it is added to something, as it is where
+// it passes through memory (the compiler would contract the pair to an fma)
+template <typename R>
+OFX_DEV cpx<R> wv_rounded(cpx<R> v) {
+#ifndef OFX_EMU
+  asm("" : "+v"(v.x), "+v"(v.y));
+#endif
+  return v;
+}
+
+// The general kernel's products by their form; OFX_SIZED (a translation unit
+// of kernels with fixed grid splits) writes the forms out.
+#ifdef OFX_SIZED
+#define OFX_MUL wv_mul
+#define OFX_MULQ wv_mulq
+#define OFX_MULC wv_mulc
+#else
+#define OFX_MUL cmul
+#define OFX_MULQ cmul
+#define OFX_MULC cmulc
+#endif
+
 // ------------------------------------------------------------------------
 // Batched Stockham FFT in LDS.  nseq sequences of length L = 2^lg, element e
 // of sequence q at buf[q*ss + e]: radix-4 passes (one radix-2 pass for odd
@@ -268,13 +339,13 @@ OFX_DEV cpx<R>* lds_fft(cpx<R>* in, cpx<R>* out, int lg, int nseq, int ss, const
         if (Ns > 1) {
           C w1 = tp[k], w2 = tp[Ns + k], w3 = tp[2 * Ns + k];
           if (SIGN > 0) {
-            v1 = cmulc(v1, w1);
-            v2 = cmulc(v2, w2);
-            v3 = cmulc(v3, w3);
+            v1 = OFX_MULC(v1, w1);
+            v2 = OFX_MULC(v2, w2);
+            v3 = OFX_MULC(v3, w3);
           } else {
-            v1 = cmul(v1, w1);
-            v2 = cmul(v2, w2);
-            v3 = cmul(v3, w3);
+            v1 = OFX_MULQ(v1, w1);
+            v2 = OFX_MULQ(v2, w2);
+            v3 = OFX_MULQ(v3, w3);
           }
         }
         C s02 = cadd(v0, v2), d02 = csub(v0, v2), s13 = cadd(v1, v3), d13 = csub(v1, v3);
@@ -740,7 +811,12 @@ struct Geo {
 template <typename R>
 OFX_DEV cpx<R> fourstep_tw(const Geo<R>& g, int m) {
   const cpx<double> a = g.twq[m >> g.lg1], b = g.twr[m & (g.n1 - 1)];
+#ifdef OFX_SIZED
+  const cpx<double> f = wv_mulq(a, b);
+  return mkc<R>((R)f.x, (R)f.y);
+#else
   return mkc<R>((R)(a.x * b.x - a.y * b.y), (R)(a.x * b.y + a.y * b.x));
+#endif
 }
 
 template <typename R>
@@ -752,7 +828,7 @@ OFX_DEV int gidx(const Geo<R>& g, int lc, int r) {
 template <typename R>
 OFX_DEV cpx<R> wt_at(const Geo<R>& g, int lc, int r) {
   const int j = gidx(g, lc, r);
-  return cmul(g.wh[j >> g.lg1], g.wl[j & (g.n1 - 1)]);
+  return OFX_MULQ(g.wh[j >> g.lg1], g.wl[j & (g.n1 - 1)]);
 }
 
 // relative angular frequency of FFT-order bin k
@@ -787,7 +863,7 @@ OFX_DEV cpx<R>* fwd_cols_to_t1(const Geo<R>& g, cpx<R>* src, cpx<R>* other, u64*
     const int cl = idx & (g.W - 1), k2 = idx >> g.lgW;
     const int c = g.c0 + cl;
     C v = res[cl * g.sT + k2];
-    v = cmul(v, fourstep_tw(g, c * k2));
+    v = OFX_MUL(v, fourstep_tw(g, c * k2));
     const TagPtr t = tp_plane<C>(g.plain, t1, g.n, t1_index(g, c, k2));
     TT::put(const_cast<u64*>(t.p), t.ws, t.plain, v, tag);
   }
@@ -912,7 +988,7 @@ OFX_DEV cpx<R>* rows_inv_to_t2(const Geo<R>& g, cpx<R>* src, cpx<R>* other, u64*
     const int k2l = idx & (g.Rr - 1), c = idx >> g.lgR;
     const int k2 = g.k20 + k2l;
     C v = res[k2l * g.sF + c];
-    v = cmulc(v, fourstep_tw(g, c * k2));
+    v = OFX_MULC(v, fourstep_tw(g, c * k2));
     const TagPtr t = tp_plane<C>(g.plain, t2, g.n, t2_index(g, c, k2));
     TT::put(const_cast<u64*>(t.p), t.ws, t.plain, v, tag);
   }
@@ -1193,9 +1269,11 @@ OFX_DEV int rk23_pass(const LaunchArgs& a, const ClusterDesc& cd, const InstDesc
 #endif
 
 // ------------------------------------------------------------------------
-// One instance: single pass (trips == 0) or round trips.
+// One instance: single pass (trips == 0) or round trips.  LG1, LG2: the grid's
+// split, fixed at compile time, of a launch without RK23 (0: read from the
+// instance).
 // ------------------------------------------------------------------------
-template <typename R, int XM>
+template <typename R, int XM, int LG1 = 0, int LG2 = 0>
 OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const InstDesc& d,
                           int rank, cpx<R>* lds, double* red, int* sflag,
                           SyncState& sy OFX_RKL_PARAM) {
@@ -1204,12 +1282,13 @@ OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const Inst
   // converged in an earlier launch (and not rewritten since): nothing to do
   if (a.conv_tol > 0.0 && a.trips > 0 && d.status[0] == ST_CONVERGED) return;
   Geo<R> g;
-  g.n = d.n;
-  g.n1 = d.n1;
-  g.n2 = d.n2;
-  g.lg1 = d.lg1;
-  g.lg2 = d.lg2;
-  g.lgn = d.lg1 + d.lg2;
+  constexpr bool FIXED = LG1 > 0;
+  g.lg1 = FIXED ? LG1 : d.lg1;
+  g.lg2 = FIXED ? LG2 : d.lg2;
+  g.lgn = g.lg1 + g.lg2;
+  g.n = FIXED ? 1 << (LG1 + LG2) : d.n;
+  g.n1 = FIXED ? 1 << LG1 : d.n1;
+  g.n2 = FIXED ? 1 << LG2 : d.n2;
   g.Cn = cd.C;
   g.lgC = 0;
   while ((1 << g.lgC) < g.Cn) g.lgC++;
@@ -1218,7 +1297,7 @@ OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const Inst
   g.lgW = g.lg1 - g.lgC;
   g.Rr = g.n2 >> g.lgC;
   g.lgR = g.lg2 - g.lgC;
-  g.HW = cd.halo;
+  g.HW = FIXED ? 2 : cd.halo;
   g.LC = g.W + 2 * g.HW;
   g.sT = g.n2 + 1;
   g.sF = g.n1 + 1;
@@ -1243,7 +1322,7 @@ OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const Inst
     // q < n2, and exp(-2 pi i r / n), r < n1; their product is rounded once,
     // as a table entry would be); then the own columns' absorber factors
     // ((lc - HW) * n2 + r, W n2 reals)
-    C* twl = lds + (d.method == METHOD_RK23 ? 5 : 3) * bs;
+    C* twl = lds + (!FIXED && d.method == METHOD_RK23 ? 5 : 3) * bs;
     const C* twg = (const C*)a.twiddle;
     const C* wtg = (const C*)d.wt;
     const int s1 = a.nmax >> d.lg1, s2 = a.nmax >> d.lg2;
@@ -1348,7 +1427,7 @@ OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const Inst
     // thread's own program order already orders its clear, writes and copy.
     if (a.trips > 0 && rank == 0 && d.stepmods)
       for (int j = OFX_TID; j < nsteps; j += OFX_NT) gl(d.stepmods)[j] = 0.0f;
-    if (d.method == METHOD_RK23) {
+    if (!FIXED && d.method == METHOD_RK23) {
       status = rk23_pass<R, MP, XM>(a, OFX_RK23_CD, d, g, rank, red, sy, breg, areg, trip_att,
                                     trip_acc);
       attempts += trip_att;
@@ -1370,46 +1449,84 @@ OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const Inst
       // exp(i*(w0 t_j - bdwz)) = wt[j] * exp(-i*bdwz); bdwz reduced in FP64
       const C eb0 = expi(-bdwz0, R(0));
       const C eb1 = expi(-bdwz1, R(0));
-      // Stage 1: K1 on columns 1..LC-2.  Each point evaluates the nonlinear
-      // term at itself and its two neighbours j+-1 (the central difference of
-      // NEE_CPU.m:104) instead of staging the term through LDS: three cheap
-      // evaluations instead of a workgroup barrier and an LDS round trip.
-      for (int idx = OFX_TID; idx < (g.LC - 2) * n2; idx += OFX_NT) {
-        const int lc = 1 + (idx >> g.lg2), r = idx & (n2 - 1);
-        const int p = lc * g.sT + r;
-        const C v = A0[p];
-        if (lc >= g.HW && lc < g.HW + g.W && !(isfinite((double)v.x) && isfinite((double)v.y)))
-          bad = 1;
-        const C nc = nl_term_e<R>(v, cmul(wt_at(g, lc, r), eb0));
-        const C nu = nl_term_e<R>(A0[p + g.sT], cmul(wt_at(g, lc + 1, r), eb0));
-        const C nd = nl_term_e<R>(A0[p - g.sT], cmul(wt_at(g, lc - 1, r), eb0));
-        K[p] = k_term<R>(nc, nu, nd, gk, cc);
-      }
-      OFX_SYNC();
-      // Stage 2 on own columns: K2 from NL(A1 = A0 + K1) at j and j+-1, the
-      // corrector E = A0 + K1/2 + K2/2, the error quotient and the absorber.
-      // E goes to X (neighbours still read K1).
       double lmax = -1.0;
-      auto corrector = [&](int idx, R f) {
-        const int lc = g.HW + (idx >> g.lg2), r = idx & (n2 - 1);
-        const int p = lc * g.sT + r;
-        const C k1 = K[p];
-        const C a0 = A0[p];
-        const C a1 = cadd(a0, k1);
-        const C nc = nl_term_e<R>(a1, cmul(wt_at(g, lc, r), eb1));
-        const C nu = nl_term_e<R>(cadd(A0[p + g.sT], K[p + g.sT]), cmul(wt_at(g, lc + 1, r), eb1));
-        const C nd = nl_term_e<R>(cadd(A0[p - g.sT], K[p - g.sT]), cmul(wt_at(g, lc - 1, r), eb1));
-        const C k2 = k_term<R>(nc, nu, nd, gk, cc);
-        C e = cadd(cadd(a0, cscale(k1, R(0.5))), cscale(k2, R(0.5)));
-        const double ex = (double)e.x - (double)a1.x, ey = (double)e.y - (double)a1.y;
-        const double err = sqrt(ex * ex + ey * ey) /
-                           (sqrt((double)e.x * (double)e.x + (double)e.y * (double)e.y) + 1.0);
-        if (err > lmax) lmax = err;
-        if (f != R(1)) e = cscale(e, f);
-        X[p] = e;
-      };
-      for (int idx = OFX_TID; idx < g.W * n2; idx += OFX_NT)
-        corrector(idx, g.ab[idx]);
+      if constexpr (FIXED) {
+        // Both stages in one pass: a thread takes 4 columns of one row with two
+        // neighbours on each side (see ofx_wave_impl.h), 4.5 evaluations of the
+        // nonlinear term a point instead of 6 and one barrier less.
+        constexpr int S = 4;
+        for (int idx = OFX_TID; idx < (g.W >> 2) * n2; idx += OFX_NT) {
+          const int s0 = (idx >> g.lg2) * S, r = idx & (n2 - 1);
+          C x[S + 4], f[S + 4], k1[S + 4], wt[S + 4];
+#pragma unroll
+          for (int i = 0; i < S + 4; i++) {
+            x[i] = A0[(s0 + i) * g.sT + r];
+            wt[i] = wt_at(g, s0 + i, r);
+            f[i] = wv_nl(x[i], wv_mul(wt[i], eb0));
+          }
+#pragma unroll
+          for (int i = 1; i < S + 3; i++)
+            k1[i] = wv_rounded(k_term<R>(f[i], f[i + 1], f[i - 1], gk, cc));
+#pragma unroll
+          for (int i = 1; i < S + 3; i++) f[i] = wv_nl(cadd(x[i], k1[i]), wv_mul(wt[i], eb1));
+#pragma unroll
+          for (int i = 2; i < S + 2; i++) {
+            if (!(isfinite((double)x[i].x) && isfinite((double)x[i].y))) bad = 1;
+            const C a1 = cadd(x[i], k1[i]);
+            // (the term of a column itself has the other rounding of exp(i th))
+            const C k2 = k_term<R>(wv_nl(a1, wv_mulq(wt[i], eb1)), f[i + 1], f[i - 1], gk, cc);
+            C e = cadd(cadd(x[i], cscale(k1[i], R(0.5))), cscale(k2, R(0.5)));
+            const double ex = (double)e.x - (double)a1.x, ey = (double)e.y - (double)a1.y;
+            const double err = sqrt(ex * ex + ey * ey) /
+                               (sqrt((double)e.x * (double)e.x + (double)e.y * (double)e.y) + 1.0);
+            if (err > lmax) lmax = err;
+            const int c = s0 + i - 2;
+            const R fa = g.ab[(c << g.lg2) + r];
+            if (fa != R(1)) e = cscale(e, fa);
+            X[(g.HW + c) * g.sT + r] = e;
+          }
+        }
+      } else {
+        // Stage 1: K1 on columns 1..LC-2.  Each point evaluates the nonlinear
+        // term at itself and its two neighbours j+-1 (the central difference of
+        // NEE_CPU.m:104) instead of staging the term through LDS: three cheap
+        // evaluations instead of a workgroup barrier and an LDS round trip.
+        for (int idx = OFX_TID; idx < (g.LC - 2) * n2; idx += OFX_NT) {
+          const int lc = 1 + (idx >> g.lg2), r = idx & (n2 - 1);
+          const int p = lc * g.sT + r;
+          const C v = A0[p];
+          if (lc >= g.HW && lc < g.HW + g.W && !(isfinite((double)v.x) && isfinite((double)v.y)))
+            bad = 1;
+          const C nc = nl_term_e<R>(v, cmul(wt_at(g, lc, r), eb0));
+          const C nu = nl_term_e<R>(A0[p + g.sT], cmul(wt_at(g, lc + 1, r), eb0));
+          const C nd = nl_term_e<R>(A0[p - g.sT], cmul(wt_at(g, lc - 1, r), eb0));
+          K[p] = k_term<R>(nc, nu, nd, gk, cc);
+        }
+        OFX_SYNC();
+        // Stage 2 on own columns: K2 from NL(A1 = A0 + K1) at j and j+-1, the
+        // corrector E = A0 + K1/2 + K2/2, the error quotient and the absorber.
+        // E goes to X (neighbours still read K1).
+        auto corrector = [&](int idx, R f) {
+          const int lc = g.HW + (idx >> g.lg2), r = idx & (n2 - 1);
+          const int p = lc * g.sT + r;
+          const C k1 = K[p];
+          const C a0 = A0[p];
+          const C a1 = cadd(a0, k1);
+          const C nc = nl_term_e<R>(a1, cmul(wt_at(g, lc, r), eb1));
+          const C nu = nl_term_e<R>(cadd(A0[p + g.sT], K[p + g.sT]), cmul(wt_at(g, lc + 1, r), eb1));
+          const C nd = nl_term_e<R>(cadd(A0[p - g.sT], K[p - g.sT]), cmul(wt_at(g, lc - 1, r), eb1));
+          const C k2 = k_term<R>(nc, nu, nd, gk, cc);
+          C e = cadd(cadd(a0, cscale(k1, R(0.5))), cscale(k2, R(0.5)));
+          const double ex = (double)e.x - (double)a1.x, ey = (double)e.y - (double)a1.y;
+          const double err = sqrt(ex * ex + ey * ey) /
+                             (sqrt((double)e.x * (double)e.x + (double)e.y * (double)e.y) + 1.0);
+          if (err > lmax) lmax = err;
+          if (f != R(1)) e = cscale(e, f);
+          X[p] = e;
+        };
+        for (int idx = OFX_TID; idx < g.W * n2; idx += OFX_NT)
+          corrector(idx, g.ab[idx]);
+      }
       // the workgroup's error maximum (+inf for a non-finite field): each
       // wave's before the barrier, then one record for the whole member, so
       // the cluster reads C records instead of C times the waves
@@ -1474,7 +1591,7 @@ OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const Inst
         C v = F[k2l * g.sF + k1];
         const C ph = expi(-beta * s_used, R(0));
         const R am = al == R(1) ? R(1) : (al == R(0) ? R(0) : (R)pow(al, (R)s_used));
-        v = cscale(cmul(v, ph), am);
+        v = cscale(OFX_MUL(v, ph), am);
         F[k2l * g.sF + k1] = v;
         if (apft) {
           OFX_GLOBAL C* ap = gl(apft);
@@ -1551,7 +1668,7 @@ OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const Inst
         C v = F[k2l * g.sF + k1];
         xesd[kk] += (double)v.x * (double)v.x + (double)v.y * (double)v.y;
         if (hist) hist[kk] = v;
-        C o = cmul(v, ocm[kk]);
+        C o = OFX_MULQ(v, ocm[kk]);
         const double S = (double)o.x * (double)o.x + (double)o.y * (double)o.y;
         if (have_prev) {
           C op = ocs[kk];
@@ -1562,8 +1679,8 @@ OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const Inst
         acc[2] += S;
         ocs[kk] = o;
         esd[kk] += S;  // each kk belongs to one thread of one member
-        C m = cmul(cav[kk], expi(-d.delay * dw_of(kk, n, dt), R(0)));
-        F[k2l * g.sF + k1] = cadd(cmul(v, m), pump ? pump[kk] : mkc<R>(R(0), R(0)));
+        C m = OFX_MUL(cav[kk], expi(-d.delay * dw_of(kk, n, dt), R(0)));
+        F[k2l * g.sF + k1] = cadd(OFX_MUL(v, m), pump ? pump[kk] : mkc<R>(R(0), R(0)));
       }
       OFX_SYNC();
       const unsigned xc2 = ++sy.nx, tagc2 = sy.base + xc2;
@@ -1661,7 +1778,10 @@ OFX_DEV void member_end(const ClusterDesc& cd, const SyncState& sy) {
 }
 
 // (with OFX_RKL, cdl: workgroup-shared storage for the descriptor's copy)
-template <typename R, int XM>
+// SIZED: Heun instances only; grids of 2^12 to 2^16 points in their default
+// split run code with the split fixed (about half of the instructions of a
+// pass form indices and addresses otherwise).
+template <typename R, int XM, bool SIZED = false>
 OFX_DEV void cluster_main(const LaunchArgs& a, int wg, cpx<R>* lds, double* red,
                           int* sflag OFX_CDL_PARAM) {
   const int ci = a.wg_cluster[wg];
@@ -1677,7 +1797,20 @@ OFX_DEV void cluster_main(const LaunchArgs& a, int wg, cpx<R>* lds, double* red,
   member_begin(a, cd, wg, rank, sflag, sy);
   for (int ii = 0; ii < cd.n_inst; ii++) {
     const int id = a.inst_order[cd.first_inst + ii];
-    run_instance<R, XM>(a, cd, a.inst[id], rank, lds, red, sflag, sy OFX_RKL_ARG);
+    const InstDesc& d = a.inst[id];
+    if constexpr (SIZED) {
+      // (a member of 4 columns or more)
+      switch (d.n1 >= 4 * cd.C ? uniform(d.lg1 * 16 + d.lg2) : 0) {
+        case 0x66: run_instance<R, XM, 6, 6>(a, cd, d, rank, lds, red, sflag, sy OFX_RKL_ARG); break;
+        case 0x76: run_instance<R, XM, 7, 6>(a, cd, d, rank, lds, red, sflag, sy OFX_RKL_ARG); break;
+        case 0x77: run_instance<R, XM, 7, 7>(a, cd, d, rank, lds, red, sflag, sy OFX_RKL_ARG); break;
+        case 0x87: run_instance<R, XM, 8, 7>(a, cd, d, rank, lds, red, sflag, sy OFX_RKL_ARG); break;
+        case 0x88: run_instance<R, XM, 8, 8>(a, cd, d, rank, lds, red, sflag, sy OFX_RKL_ARG); break;
+        default: run_instance<R, XM>(a, cd, d, rank, lds, red, sflag, sy OFX_RKL_ARG);
+      }
+    } else {
+      run_instance<R, XM>(a, cd, d, rank, lds, red, sflag, sy OFX_RKL_ARG);
+    }
     if (flag_load(cd.abort_flag)) break;
   }
   member_end(cd, sy);

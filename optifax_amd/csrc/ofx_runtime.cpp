@@ -341,6 +341,12 @@ int wave_block(const ofx_pass_params& p, int n1, int C, size_t csz, int lds_max)
   return p.n / C <= 1024 && wave_points(p, n1, C, block, csz, lds_max) ? block : 0;
 }
 
+// XMODE_SIZED where a launch of the general kernel without RK23 can have it (32
+// cavities of 2^14 to 2^16 points 76.9 ms a trip, without it 87.8).
+int sized_mode(int exchange, int block) {
+  return exchange == 1 && block == XMODE_SIZED_BLOCK ? (int)XMODE_SIZED : 0;
+}
+
 // Launch mode of the wave kernel with this many points a thread (wave_points):
 // the kernel with the default geometry fixed where this is it for every
 // instance (2^8 2.6 against 4.1 us per step, 2^12 5.8 against 7.3, 2^15 8.1
@@ -589,9 +595,11 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
   r->inst_C.resize(n_inst);
   r->inst_n1.resize(n_inst);
   int nmax = 0;
-  bool all_rk23 = n_inst > 0;
-  for (int i = 0; i < n_inst; i++)
+  bool all_rk23 = n_inst > 0, all_heun = n_inst > 0;
+  for (int i = 0; i < n_inst; i++) {
     all_rk23 = all_rk23 && specs[i].pass.method == OFX_METHOD_RK23;
+    all_heun = all_heun && specs[i].pass.method == OFX_METHOD_HEUN;
+  }
   // (a launch runs one kernel: RK23 beside Heun is the general one's)
   auto waves = [&](int i) { return all_rk23 || specs[i].pass.method == OFX_METHOD_HEUN; };
   for (int i = 0; i < n_inst; i++) {
@@ -641,7 +649,9 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
     r->xmode = points ? wave_mode(points, r->block, same ? ilog2i(specs[0].pass.n) : 0, r->inst_n1[0],
                                   r->inst_C[0], specs[0].pass.method, r->csz)
                       : exchange_mode(exchange, cmin);
-    if (all_rk23) r->xmode |= XMODE_RK23_LDS;
+    r->xmode |= all_rk23              ? (int)XMODE_RK23_LDS
+                : all_heun && !points ? sized_mode(r->xmode, r->block)
+                                      : 0;
     const int bpc = be_blocks_per_cu(ctx->be, precision, r->xmode, r->block, r->lds);
     if (bpc < 1)
       return fail(ctx, OFX_E_ARG, "kernel cannot launch with block=%d and %zu bytes of LDS", r->block,
@@ -1390,7 +1400,9 @@ extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params*
   const int points = wblock ? wave_points(*p, n1, C, block, 8, ctx->info.lds_max) : 0;
   const int xmode = points ? wave_mode(points, block, ilog2i(n), n1, C, method, 8) |
                                  (method == OFX_METHOD_RK23 ? (int)XMODE_RK23_LDS : 0)
-                           : exchange_mode(0, C);
+                           : exchange_mode(0, C) | (method == OFX_METHOD_HEUN
+                                                        ? sized_mode(exchange_mode(0, C), block)
+                                                        : 0);
   const size_t lds = points ? wave_lds_bytes(n1, n2, C, method, 8) : lds_bytes_for(n1, n2, C, method, 8);
   const int bpc = be_blocks_per_cu(ctx->be, OFX_F32, xmode, block, lds);
   if (bpc < 1)

@@ -51,63 +51,6 @@ OFX_DEV void wv_order() {
 #endif
 }
 
-// The products' fused forms are written out here: left to the compiler, which
-// of a sum's two products is rounded first depends on the code around it, and
-// these are the forms that the general kernel's code has (so that both give
-// the same bits).
-template <typename R>
-OFX_DEV R wv_fma(R a, R b, R c) {
-#ifdef OFX_EMU
-  return a * b + c;   // (the emulation's host code fuses nothing)
-#else
-  if constexpr (sizeof(R) == 4)
-    return __builtin_fmaf(a, b, c);
-  else
-    return __builtin_fma(a, b, c);
-#endif
-}
-// a b, the imaginary part's a.y b.x rounded first (FP64: the other one)
-template <typename R>
-OFX_DEV cpx<R> wv_mul(cpx<R> a, cpx<R> b) {
-  if constexpr (sizeof(R) == 8)
-    return mkc<R>(wv_fma(a.x, b.x, -(a.y * b.y)), wv_fma(a.y, b.x, a.x * b.y));
-  return mkc<R>(wv_fma(a.x, b.x, -(a.y * b.y)), wv_fma(a.x, b.y, a.y * b.x));
-}
-// a b, the imaginary part's a.x b.y rounded first
-template <typename R>
-OFX_DEV cpx<R> wv_mulq(cpx<R> a, cpx<R> b) {
-  return mkc<R>(wv_fma(a.x, b.x, -(a.y * b.y)), wv_fma(a.y, b.x, a.x * b.y));
-}
-// a conj(b)
-template <typename R>
-OFX_DEV cpx<R> wv_mulc(cpx<R> a, cpx<R> b) {
-  return mkc<R>(wv_fma(a.x, b.x, a.y * b.y), wv_fma(a.y, b.x, -(a.x * b.y)));
-}
-// |a|^2 in FP64
-template <typename R>
-OFX_DEV double wv_abs2(cpx<R> a) {
-  const double x = a.x, y = a.y;
-  return wv_fma(x, x, y * y);
-}
-// nl_term_e
-template <typename R>
-OFX_DEV cpx<R> wv_nl(cpx<R> A, cpx<R> e) {
-  const R yy = A.y * A.y;
-  const R a2 = R(2) * wv_fma(A.x, A.x, yy), sx = wv_fma(A.x, A.x, -yy), sy = R(2) * A.x * A.y;
-  const R im = sizeof(R) == 8 ? wv_fma(sy, e.x, sx * e.y) : wv_fma(sx, e.y, sy * e.x);
-  return mkc<R>(wv_fma(a2, e.x, wv_fma(sx, e.x, -(sy * e.y))), wv_fma(-a2, e.y, im));
-}
-
-// A product that is rounded before it is added to something, as it is where
-// it passes through memory (the compiler would contract the pair to an fma)
-template <typename R>
-OFX_DEV cpx<R> wv_rounded(cpx<R> v) {
-#ifndef OFX_EMU
-  asm("" : "+v"(v.x), "+v"(v.y));
-#endif
-  return v;
-}
-
 // State of one thread.  On the device one object per thread, in registers; in
 // the emulation an array that each phase walks.
 template <typename R, int S, int HW = 2>

@@ -83,12 +83,12 @@ int be_blocks_per_cu(Backend*, int, int, int, size_t lds) { return lds <= 160 * 
 // the RK23 variant's workgroup body (ofx_backend_emu_rkl.cpp)
 void (*emu_rkl_fn(int precision, int xmode))(const LaunchArgs*, int, size_t);
 
-template <typename R, int XM>
+template <typename R, int XM, bool SIZED = false>
 static void run_wg(const LaunchArgs* a, int wg, size_t lds) {
   std::vector<unsigned char> mem(lds + 64);
   double red[64];
   int sflag[4];
-  cluster_main<R, XM>(*a, wg, reinterpret_cast<cpx<R>*>(mem.data()), red, sflag);
+  cluster_main<R, XM, SIZED>(*a, wg, reinterpret_cast<cpx<R>*>(mem.data()), red, sflag);
 }
 
 // the wave kernel: a workgroup's threads are walked phase by phase
@@ -159,7 +159,10 @@ int be_launch(Backend* b, const LaunchArgs& a, int precision, int xmode, int gri
                             ? (precision == OFX_F64 ? wave_fn<double, 4>(pts) : wave_fn<float, 4>(pts))
                             : (precision == OFX_F64 ? wave_fn<double, 2>(pts) : wave_fn<float, 2>(pts)),
                         &a, wg, lds);
-      } else if (xmode & XMODE_RK23_LDS)
+      } else if (xmode & XMODE_SIZED)
+        th.emplace_back(precision == OFX_F64 ? run_wg<double, XM_BARRIER, true>
+                                             : run_wg<float, XM_BARRIER, true>, &a, wg, lds);
+      else if (xmode & XMODE_RK23_LDS)
         th.emplace_back(emu_rkl_fn(precision, xmode & 1), &a, wg, lds);
       else if (precision == OFX_F64)
         th.emplace_back(bar ? run_wg<double, XM_BARRIER> : run_wg<double, XM_TAGS>, &a, wg, lds);
