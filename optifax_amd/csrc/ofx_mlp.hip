@@ -579,6 +579,7 @@ struct ofx_mlp {
   long long adam_t = 0;
   unsigned char* stage = nullptr;  // STAGES pinned buffers of STAGE_BYTES (made on first use)
   hipEvent_t stage_ev[STAGES] = {};
+  std::mutex stage_mu;             // one result at a time passes through them
   hipStream_t stream = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
   double last_ms = 0.0;
@@ -795,8 +796,11 @@ static int check_batch(ofx_mlp* m, int B) {
 
 // Brings a result of `bytes` to host memory through the pinned buffers:
 // fill(buf, at, len) enqueues the transfer of its bytes [at, at + len) to buf.
+// The buffers and events are the handle's: threads that read one handle take
+// turns, or one would copy out what another's transfer has put there.
 template <typename Fill>
 static int deliver(ofx_mlp* m, void* dst, size_t bytes, Fill fill) {
+  std::lock_guard<std::mutex> turn(m->stage_mu);
   for (hipEvent_t& e : m->stage_ev)
     if (!e) MCHK(m, hipEventCreateWithFlags(&e, hipEventDisableTiming));
   if (!m->stage)
@@ -835,7 +839,9 @@ static int deliver(ofx_mlp* m, void* dst, size_t bytes, Fill fill) {
   work(0);
   for (std::thread& t : th) t.join();
   const hipError_t e = (hipError_t)failed.load();
-  return e == hipSuccess ? OFX_OK : mlp_fail(m, "result transfer", e);
+  if (e == hipSuccess) return OFX_OK;
+  (void)hipStreamSynchronize(m->stream);   // nothing in flight to the buffers
+  return mlp_fail(m, "result transfer", e);
 }
 
 // A parameter-shaped device vector to host memory in the public layout.
