@@ -103,6 +103,9 @@ zsum_kernel(int n_out, const double* __restrict__ dk, int n_run, const double* _
   const double th = reduce_2pi(k * dz);
   double s_half, c_half;
   sincos_cw(0.5 * th, s_half, c_half);
+  // Below 1e-18 the series factor of a run of m < 2^31 samples is m to
+  // rounding; formed with that sine, terms of very small dk would underflow.
+  if (fabs(s_half) < 1e-18) s_half = 0.0;
   double ar = 0.0, ai = 0.0;
   // the series factor depends on the run length only: kept while consecutive
   // runs share it (a uniform grating has one or two lengths)
