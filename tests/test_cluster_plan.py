@@ -1,0 +1,56 @@
+"""Cluster sizes follow the kernel that runs.  A launch that the wave kernel
+cannot take (RK23 beside Heun, a workgroup size that is no power of two, a grid
+that it does not fit) has the general kernel's cluster sizes, which the counter
+barrier's launches always have."""
+import os
+
+import pytest
+
+from cases import opo_case
+from optifax_amd.solver import Context, OPOBatch
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def ctx256():
+    path = os.path.join(ROOT, "tests", "emu", "libofx_emu.so")
+    if not os.path.exists(path):
+        pytest.skip("emulation library not built")
+    old = os.environ.get("OFX_EMU_CUS")
+    os.environ["OFX_EMU_CUS"] = "256"
+    ctx = Context(0, lib_path=path)
+    if old is None:
+        del os.environ["OFX_EMU_CUS"]
+    else:
+        os.environ["OFX_EMU_CUS"] = old
+    yield ctx
+    ctx.close()
+
+
+def clusters(ctx, grids, precision="single", tune=None):
+    insts = []
+    for n, method in grids:
+        _, b = opo_case(n=n, window=3e-12 * (n / 512) ** 0.5, length=6e-6)
+        insts.append(dict(solver=b["solver"], field0=b["ops"]["field0"], method=method))
+    run = OPOBatch(insts, precision=precision, ctx=ctx, tune=tune)
+    out = [run.geometry(i)["cluster"] for i in range(len(insts))], run.geometry(0)["lds_bytes"]
+    run.close()
+    return out
+
+
+@pytest.mark.parametrize("precision", ["single", "double"])
+@pytest.mark.parametrize("n", [512, 1024, 4096])
+@pytest.mark.parametrize("pairs", [1, 4])
+def test_heun_beside_rk23(ctx256, n, pairs, precision):
+    grids = [(n, "heun"), (n, "rk23")] * pairs
+    assert clusters(ctx256, grids, precision) == \
+        clusters(ctx256, grids, precision, dict(exchange="barrier"))
+
+
+@pytest.mark.parametrize("precision", ["single", "double"])
+@pytest.mark.parametrize("method", ["heun", "rk23"])
+@pytest.mark.parametrize("n", [512, 1024, 4096])
+def test_odd_workgroup_size(ctx256, n, method, precision):
+    assert clusters(ctx256, [(n, method)], precision, dict(block=192)) == \
+        clusters(ctx256, [(n, method)], precision, dict(block=192, exchange="barrier"))
