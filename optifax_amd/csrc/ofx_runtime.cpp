@@ -628,9 +628,18 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
     }
     if (int st = plan_block(ctx, tune, cmin, wblock, &r->block)) return st;
     // the wave kernel when it suits every instance (a caller that asks for the
-    // tagged exchange has it wherever it can run)
+    // tagged exchange has it wherever it can run).  With FP64 fields and more
+    // than 256 threads it spills, and in clusters of several workgroups the
+    // general kernel is the faster one (2^15 at 64 23.5 against 16.6 us per
+    // step, at 128 26.4 against 16.2; 2^12 at 16 17.7 against 12.5; alone 2^9
+    // 9.4, general 11.9): then only where the caller gives both the exchange and
+    // the threads.
+    const int cmax = *std::max_element(r->inst_C.begin(), r->inst_C.end());
+    const bool spills = precision == OFX_F64 && r->block > 256 && cmax > 1;
+    const bool wave = exchange == 1 ? !spills || (tune && tune->block)
+                                    : exchange == 0 && wblock && !spills;
     int points = 0;
-    for (int i = 0; i < n_inst && (exchange == 1 || (exchange == 0 && wblock)); i++) {
+    for (int i = 0; i < n_inst && wave; i++) {
       const int w = waves ? wave_points(specs[i].pass, r->inst_n1[i], r->inst_C[i], r->block,
                                         r->csz, ctx->info.lds_max)
                           : 0;

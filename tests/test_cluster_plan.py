@@ -54,3 +54,33 @@ def test_heun_beside_rk23(ctx256, n, pairs, precision):
 def test_odd_workgroup_size(ctx256, n, method, precision):
     assert clusters(ctx256, [(n, method)], precision, dict(block=192)) == \
         clusters(ctx256, [(n, method)], precision, dict(block=192, exchange="barrier"))
+
+
+@pytest.mark.parametrize("method", ["heun", "rk23"])
+@pytest.mark.parametrize("n", [4096, 8192, 32768])
+def test_f64_workgroups_of_512_threads(ctx256, n, method):
+    """FP64 fields in clusters of 512-thread workgroups: the general kernel (its
+    workspace and clusters), also with the tagged exchange unless the caller
+    gives the threads too."""
+    general = clusters(ctx256, [(n, method)], "double", dict(block=512, exchange="barrier"))
+    assert clusters(ctx256, [(n, method)], "double", dict(block=512)) == general
+    assert clusters(ctx256, [(n, method)], "double",
+                    dict(block=512, cluster=general[0][0])) == general
+    both = dict(block=512, exchange="tags", cluster=general[0][0])
+    assert clusters(ctx256, [(n, method)], "double", both)[1] != general[1]
+
+
+def test_f64_large_shares_with_tags(ctx256):
+    """Shares above the wave kernel's default: the tagged exchange alone brings
+    the general kernel (FP64, 512 threads)."""
+    many = [(32768, "heun")] * 16
+    assert clusters(ctx256, many, "double", dict(exchange="tags")) == \
+        clusters(ctx256, many, "double", dict(exchange="barrier"))
+
+
+def test_f64_one_workgroup_of_512_threads(ctx256):
+    """One workgroup without an exchange keeps the wave kernel."""
+    got = clusters(ctx256, [(512, "heun")], "double", dict(block=512))
+    general = clusters(ctx256, [(512, "heun")], "double",
+                       dict(block=512, cluster=1, exchange="barrier"))
+    assert got[0] == [1] and got[1] != general[1]
