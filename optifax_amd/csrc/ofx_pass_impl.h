@@ -1451,11 +1451,14 @@ OFX_DEV void run_instance(const LaunchArgs& a, const ClusterDesc& cd, const Inst
       const C eb1 = expi(-bdwz1, R(0));
       double lmax = -1.0;
       if constexpr (FIXED) {
-        // Both stages in one pass: a thread takes 4 columns of one row with two
-        // neighbours on each side (see ofx_wave_impl.h), 4.5 evaluations of the
-        // nonlinear term a point instead of 6 and one barrier less.
-        constexpr int S = 4;
-        for (int idx = OFX_TID; idx < (g.W >> 2) * n2; idx += OFX_NT) {
+        // Both stages in one pass: a thread takes S columns of one row with two
+        // neighbours on each side (see ofx_wave_impl.h), and one barrier less.  4
+        // columns evaluate the nonlinear term 4.5 times a point instead of 6; with
+        // FP64 fields they spill 675 registers, and 2 columns (6 times, 324) are
+        // the faster: us per step on a full device, general / 4 / 2 columns, 2^13
+        // on 4 workgroups 29.1 / 30.5 / 27.3, 2^15 on 16 33.1 / 33.1 / 31.7.
+        constexpr int S = sizeof(R) == 8 ? 2 : 4;
+        for (int idx = OFX_TID; idx < (g.W / S) * n2; idx += OFX_NT) {
           const int s0 = (idx >> g.lg2) * S, r = idx & (n2 - 1);
           C x[S + 4], f[S + 4], k1[S + 4], wt[S + 4];
 #pragma unroll

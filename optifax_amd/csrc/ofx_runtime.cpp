@@ -341,10 +341,18 @@ int wave_block(const ofx_pass_params& p, int n1, int C, size_t csz, int lds_max)
   return p.n / C <= 1024 && wave_points(p, n1, C, block, csz, lds_max) ? block : 0;
 }
 
-// XMODE_SIZED where a launch of the general kernel without RK23 can have it (32
-// cavities of 2^14 to 2^16 points 76.9 ms a trip, without it 87.8).
-int sized_mode(int exchange, int block) {
-  return exchange == 1 && block == XMODE_SIZED_BLOCK ? (int)XMODE_SIZED : 0;
+// Whether the general kernel has a form with this split fixed (cluster_main's
+// cases; a member of 4 columns or more).
+bool sized_form(int n1, int n2, int C) {
+  return n1 >= 4 * C && n2 >= 64 && n1 <= 256 && (n1 == n2 || n1 == 2 * n2);
+}
+
+// XMODE_SIZED where a launch of the general kernel without RK23 can have it and
+// some instance has a form (32 cavities of 2^14 to 2^16 points 76.9 ms a trip,
+// without it 87.8; without a form FP64 2^11 takes 28.9 us per step, in the plain
+// general kernel 28.1).
+int sized_mode(int exchange, int block, bool form) {
+  return exchange == 1 && block == XMODE_SIZED_BLOCK && form ? (int)XMODE_SIZED : 0;
 }
 
 // Launch mode of the wave kernel with this many points a thread (wave_points):
@@ -647,10 +655,12 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
       if (!w) break;
     }
     bool same = true;  // one grid size and geometry throughout
+    bool form = false;
     r->lds = 0;
     for (int i = 0; i < n_inst; i++) {
       const int n = specs[i].pass.n, n1 = r->inst_n1[i], C = r->inst_C[i];
       same = same && n == specs[0].pass.n && n1 == r->inst_n1[0] && C == r->inst_C[0];
+      form = form || sized_form(n1, n / n1, C);
       const int method = specs[i].pass.method;
       r->lds = std::max(r->lds, points ? wave_lds_bytes(n1, n / n1, C, method, r->csz)
                                        : lds_bytes_for(n1, n / n1, C, method, r->csz));
@@ -659,7 +669,7 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
                                   r->inst_C[0], specs[0].pass.method, r->csz)
                       : exchange_mode(exchange, cmin);
     r->xmode |= all_rk23              ? (int)XMODE_RK23_LDS
-                : all_heun && !points ? sized_mode(r->xmode, r->block)
+                : all_heun && !points ? sized_mode(r->xmode, r->block, form)
                                       : 0;
     const int bpc = be_blocks_per_cu(ctx->be, precision, r->xmode, r->block, r->lds);
     if (bpc < 1)
@@ -1416,11 +1426,15 @@ extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params*
   if (st) return st;
   const int n2 = n / n1;
   const int points = wblock ? wave_points(*p, n1, C, block, 8, ctx->info.lds_max) : 0;
-  const int xmode = points ? wave_mode(points, block, ilog2i(n), n1, C, method, 8) |
-                                 (method == OFX_METHOD_RK23 ? (int)XMODE_RK23_LDS : 0)
-                           : exchange_mode(0, C) | (method == OFX_METHOD_HEUN
-                                                        ? sized_mode(exchange_mode(0, C), block)
-                                                        : 0);
+  int xmode = 0;
+  if (points)
+    xmode = wave_mode(points, block, ilog2i(n), n1, C, method, 8) |
+            (method == OFX_METHOD_RK23 ? (int)XMODE_RK23_LDS : 0);
+  else
+    xmode = exchange_mode(0, C) |
+            (method == OFX_METHOD_HEUN
+                 ? sized_mode(exchange_mode(0, C), block, sized_form(n1, n2, C))
+                 : 0);
   const size_t lds = points ? wave_lds_bytes(n1, n2, C, method, 8) : lds_bytes_for(n1, n2, C, method, 8);
   const int bpc = be_blocks_per_cu(ctx->be, OFX_F32, xmode, block, lds);
   if (bpc < 1)

@@ -132,11 +132,27 @@ static void (*fixed_fn(int lg))(const LaunchArgs*, int, size_t) {
   }
 }
 
+// the last launch: its mode, and every instance's grid size and cluster (for
+// tests of which kernel and schedule a launch has)
+static int g_last_xmode = -1;
+static std::vector<int> g_last_n, g_last_cluster;
+
 int be_launch(Backend* b, const LaunchArgs& a, int precision, int xmode, int grid, int block,
               size_t lds, unsigned* const* zp, const size_t* zw, int nz, unsigned* ep, int nep,
               const void* key, int replays) {
   (void)key;
   (void)block;
+  g_last_xmode = xmode;
+  g_last_n.clear();
+  g_last_cluster.clear();
+  for (int wg = 0; wg < grid; wg++) {
+    const int c = a.wg_cluster[wg];
+    if (c < 0 || a.wg_rank[wg] != 0) continue;
+    for (int i = 0; i < a.clusters[c].n_inst; i++) {
+      g_last_n.push_back(a.inst[a.inst_order[a.clusters[c].first_inst + i]].n);
+      g_last_cluster.push_back(c);
+    }
+  }
   const int reps = replays > 0 ? replays : 1;
   for (int rep = 0; rep < reps; rep++) {
     for (int i = 0; i < nz; i++) memset(zp[i], 0, zw[i] * sizeof(unsigned));
@@ -192,3 +208,12 @@ int be_widen(Backend*, double* dst, const float* src, size_t n) {
 int be_d2d(Backend*, void* dst, const void* src, size_t bytes) { memcpy(dst, src, bytes); return OFX_OK; }
 
 }  // namespace ofx
+
+extern "C" int ofx_emu_last_launch(int max, int* n, int* cluster, int* count) {
+  *count = (int)ofx::g_last_n.size();
+  for (int i = 0; i < *count && i < max; i++) {
+    n[i] = ofx::g_last_n[i];
+    cluster[i] = ofx::g_last_cluster[i];
+  }
+  return ofx::g_last_xmode;
+}
