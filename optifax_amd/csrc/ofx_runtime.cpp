@@ -390,16 +390,21 @@ int exchange_mode(int exchange, int cmin) {
   return exchange == 1 ? 0 : exchange == 2 ? 1 : (cmin >= 64 ? 0 : 1);
 }
 
-// An adaptive step's time [us] on a full device, fitted (within 10 %) to full
-// devices of 2^12 to 2^16 points at 256 to 4096 points a workgroup: general
-// kernel FP32 2^12 15.8 us at 1024 points, 34.7 at 4096; 2^16 22 and 39; FP64
-// 2^12 19.5 at 1024, 2^15 33 at 2048; wave kernel FP32 2^12 9.1 at 512, 2^15
-// 14.6 at 1024, FP64 2^12 13.2 and 2^15 20.6.  Only ratios are used.
+// An adaptive step's time [us] on a full device, for a plan's choice; only ratios
+// count.  Wave kernel with Heun, by 1024 points a workgroup (here / measured): FP32
+// 2^12 12.2 / 12.9, 2^15 14.3 / 15.0, 2^16 15.0 / 19.3; FP64 2^12 15.6 / 15.9, 2^14
+// 21.9 / 22.0, 2^15 19.5 / 20.8, 2^16 20.8 / 28.9; RK23 takes up to 25 % less than
+// this.  General kernel at 2048 points: FP32 2^12 20.7 / 19.3, 2^16 25.5 / 21.6, FP64
+// 2^13 30.6 / 27.3, 2^15 33.0 / 30.7 (its fixed splits are newer than the fit).  That
+// it leans to the wave kernel is wanted: a cluster's last instances run on a device
+// that is no longer full, where that kernel gains most.  With both fitted within
+// 10 %, 300 FP32 cavities of 2^11 took 41.1 us a step in place of 33.9, and five FP64
+// ones of 2^15 and 2^16 5.1 ms in place of 3.8.
 double step_us(const ofx_pass_params& p, int C, bool f64, bool wave) {
   const double x = ilog2i(p.n) - 14, share = (double)p.n / C;
   const bool rk23 = p.method == OFX_METHOD_RK23;
   if (wave)
-    return (rk23 ? 1.35 : 1.0) *
+    return (rk23 ? 1.35 : 1.0) * (f64 && x == 0 && share > 512 ? 1.2 : 1.0) *
            (f64 ? 13.6 + 1.3 * x + 4.5e-3 * share : 6.9 + 0.7 * x + 6.5e-3 * share);
   const double t = f64 ? 13.0 + 1.2 * x + 9.2e-3 * share
                        : 12.5 + 1.2 * x + 5.2e-3 * share + 1.7e-3 * std::max(0.0, share - 2048);

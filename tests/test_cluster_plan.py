@@ -84,3 +84,12 @@ def test_f64_one_workgroup_of_512_threads(ctx256):
     general = clusters(ctx256, [(512, "heun")], "double",
                        dict(block=512, cluster=1, exchange="barrier"))
     assert got[0] == [1] and got[1] != general[1]
+
+
+def test_f64_batch_of_16384_points(ctx256):
+    """40 FP64 instances of 2^14: a step of the wave kernel at 1024 points a
+    workgroup takes 22 us there, so three rounds of it (66) are no gain over two of
+    the general kernel (60)."""
+    many = [(16384, "heun")] * 40
+    got, lds = clusters(ctx256, many, "double")
+    assert got == [8] * 40 and lds == clusters(ctx256, many, "double", dict(exchange="barrier"))[1]
