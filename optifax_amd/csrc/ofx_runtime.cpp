@@ -630,6 +630,7 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
   for (int i = 0; i < n_inst; i++) given = given || specs[i].cluster;
   // threads, launch mode and LDS for the cluster sizes in r->inst_C
   int slots = 0;
+  bool avoid_spills = true, spilled = false;
   auto geometry = [&]() -> int {
     int cmin = 1 << 30, wblock = 0;
     for (int i = 0; i < n_inst; i++) {
@@ -648,7 +649,8 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
     // 9.4, general 11.9): then only where the caller gives both the exchange and
     // the threads.
     const int cmax = *std::max_element(r->inst_C.begin(), r->inst_C.end());
-    const bool spills = precision == OFX_F64 && r->block > 256 && cmax > 1;
+    const bool spills = avoid_spills && precision == OFX_F64 && r->block > 256 && cmax > 1;
+    spilled = spilled || spills;
     const bool wave = exchange == 1 ? !spills || (tune && tune->block)
                                     : exchange == 0 && wblock && !spills;
     int points = 0;
@@ -685,50 +687,57 @@ int ofx_opo_create(ofx_context* ctx, int precision, int n_inst, const ofx_opo_sp
   };
   const bool f64 = precision == OFX_F64;
   auto wave_runs = [&] { return (r->xmode & (XMODE_WAVE_MASK | XMODE_FIXED_MASK)) != 0; };
-  st = plan_all(waves);
-  if (!st) st = geometry();
-  if (!st && waves && !wave_runs()) {
-    // the general kernel on its own cluster sizes (with the wave kernel's a 2^9
-    // instance in workgroups of 192 threads takes 12.4 us per step instead of
-    // 11.3, RK23 14.6 instead of 12.1; 2^10 beside RK23 11.6 instead of 10.5)
-    st = plan_all(false);
+  BatchPlan plan;
+  std::vector<int> cl_C, cl_method;
+  auto schedule = [&]() -> int {
+    int st = plan_all(waves);
     if (!st) st = geometry();
+    if (waves && (st || !wave_runs())) {
+      // the general kernel on its own cluster sizes (the wave kernel's may not fit
+      // LDS there; and with them a 2^9 instance in workgroups of 192 threads takes
+      // 12.4 us per step instead of 11.3, RK23 14.6 instead of 12.1; 2^10 beside
+      // RK23 11.6 instead of 10.5)
+      st = plan_all(false);
+      if (!st) st = geometry();
+    }
+    if (st) return st;
+    // equal shares unless uneven ones promise a 5 % shorter launch
+    plan = plan_equal(n_inst, specs, r->inst_C, r->inst_n1, slots, f64, wave_runs());
+    for (bool wave : {false, true}) {
+      BatchPlan uneven;
+      if (given || !plan_uneven(n_inst, specs, r->inst_n1, ctx->info.cus, r->csz, ctx->info.lds_max,
+                                wave, &uneven) ||
+          uneven.span > 0.95 * plan.span)
+        continue;
+      r->inst_C = uneven.C;
+      if (geometry() == OFX_OK && wave_runs() == wave) plan = uneven;
+      r->inst_C = plan.C;
+    }
+    if (int st = geometry()) return st;
+    long long used = 0;
+    cl_C.clear();
+    cl_method.clear();
+    for (const auto& m : plan.members) {
+      cl_C.push_back(r->inst_C[m[0]]);
+      cl_method.push_back(specs[m[0]].pass.method);
+      used += cl_C.back();
+    }
+    if (used > slots)
+      return fail(ctx, OFX_E_ARG, "schedule needs %lld workgroups, only %d fit at once", used, slots);
+    return OFX_OK;
+  };
+  st = schedule();
+  if (st && spilled) {
+    // only the wave kernel fits
+    avoid_spills = false;
+    st = schedule();
   }
   if (st) {
     delete r;
     return st;
   }
   r->nmax = nmax;
-
-  // ---- clusters: equal shares unless uneven ones promise a 5 % shorter launch ----
-  BatchPlan plan = plan_equal(n_inst, specs, r->inst_C, r->inst_n1, slots, f64, wave_runs());
-  for (bool wave : {false, true}) {
-    BatchPlan uneven;
-    if (given || !plan_uneven(n_inst, specs, r->inst_n1, ctx->info.cus, r->csz, ctx->info.lds_max,
-                              wave, &uneven) ||
-        uneven.span > 0.95 * plan.span)
-      continue;
-    r->inst_C = uneven.C;
-    if (geometry() == OFX_OK && wave_runs() == wave) plan = uneven;
-    r->inst_C = plan.C;
-  }
-  st = geometry();
-  if (st) {
-    delete r;
-    return st;
-  }
   const std::vector<std::vector<int>>& cl_members = plan.members;
-  std::vector<int> cl_C, cl_method;
-  for (const auto& m : cl_members) {
-    cl_C.push_back(r->inst_C[m[0]]);
-    cl_method.push_back(specs[m[0]].pass.method);
-  }
-  long long used = 0;
-  for (int C : cl_C) used += C;
-  if (used > slots) {
-    delete r;
-    return fail(ctx, OFX_E_ARG, "schedule needs %lld workgroups, only %d fit at once", used, slots);
-  }
 
   // ---- XCD-aware placement: workgroup id g runs on XCD g % nxcd ----
   const int nx = std::max(1, ctx->info.nxcd);

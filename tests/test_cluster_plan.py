@@ -93,3 +93,28 @@ def test_f64_batch_of_16384_points(ctx256):
     many = [(16384, "heun")] * 40
     got, lds = clusters(ctx256, many, "double")
     assert got == [8] * 40 and lds == clusters(ctx256, many, "double", dict(exchange="barrier"))[1]
+
+
+@pytest.mark.parametrize("block", [64, 128, 192, 512])
+def test_given_threads_with_clusters_of_the_wave_kernel(ctx256, block):
+    """Shares that fit LDS in the wave kernel only: with threads that it does not
+    take, the general kernel has larger clusters of its own."""
+    many = [(16384, "rk23")] * 10
+    got, _ = clusters(ctx256, many, "double", dict(block=block))
+    assert got == clusters(ctx256, many, "double", dict(block=block, exchange="barrier"))[0]
+
+
+def test_f64_threads_that_only_the_wave_kernel_fits():
+    """512 threads given: where the general kernel's clusters do not fit the
+    device (a part of 32 CUs), the wave kernel runs."""
+    path = os.path.join(ROOT, "tests", "emu", "libofx_emu.so")
+    if not os.path.exists(path):
+        pytest.skip("emulation library not built")
+    os.environ["OFX_EMU_CUS"] = "32"
+    try:
+        ctx = Context(0, lib_path=path)
+    finally:
+        del os.environ["OFX_EMU_CUS"]
+    got = clusters(ctx, [(16384, "rk23"), (2048, "rk23")], "double", dict(block=512))
+    ctx.close()
+    assert sum(got[0]) <= 32
