@@ -1408,22 +1408,13 @@ size_t na_take(size_t& off, size_t bytes) {
 
 }  // namespace
 
-extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params* p, int batch,
-                                        float* Et, const float* alpha_w, const float* G,
-                                        int g_batch, const float* beta_op, float* ApFT,
-                                        float* stepMods, int* status) {
-  if (!ctx) return OFX_E_ARG;
-  int st = check_pass(ctx, p);
-  if (st) return st;
-  if (batch == 0) return OFX_OK;
-  if (batch < 0 || !Et || !alpha_w || !G || !beta_op)
-    return fail(ctx, OFX_E_ARG, "Et, alpha_w, G, beta_op are required and batch >= 0");
-  if (g_batch != 1 && g_batch != batch)
-    return fail(ctx, OFX_E_ARG, "G must hold NSteps or NSteps*batch values (g_batch=%d)", g_batch);
-  if (batch > NA_MAX_BATCH)
-    return fail(ctx, OFX_E_ARG, "the no-allocation pass takes at most %d instances (got %d)",
-                NA_MAX_BATCH, batch);
-  std::lock_guard<std::mutex> lock(g_na_mu);
+// The pass on checked arguments, with g_na_mu held.  waves: the wave kernel may
+// run it.  Where its larger clusters' exchange buffers do not fit the array (2^11
+// points, 16 workgroups instead of 8), the general kernel's may.
+static int noalloc_pass(ofx_context* ctx, const ofx_pass_params* p, int batch, float* Et,
+                        const float* alpha_w, const float* G, int g_batch, const float* beta_op,
+                        float* ApFT, float* stepMods, int* status, bool waves) {
+  int st = OFX_OK;
   unsigned char* base = nullptr;
   size_t cap = 0;
   if (be_scratch(ctx->be, &base, &cap))
@@ -1434,8 +1425,8 @@ extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params*
   // geometry: as ofx_opo_create plans a batch of equal instances (one
   // cluster per instance, all resident at once)
   int C = 0, n1 = 0, block = 0;
-  st = plan_instance(ctx, *p, batch, nullptr, 0, 0, 8, true, &C, &n1);
-  const int wblock = st ? 0 : wave_block(*p, n1, C, 8, ctx->info.lds_max);
+  st = plan_instance(ctx, *p, batch, nullptr, 0, 0, 8, waves, &C, &n1);
+  const int wblock = st || !waves ? 0 : wave_block(*p, n1, C, 8, ctx->info.lds_max);
   if (!st) st = plan_block(ctx, nullptr, C, wblock, &block);
   if (st) return st;
   const int n2 = n / n1;
@@ -1514,6 +1505,9 @@ extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params*
   const size_t o_beta = na_take(off, 8 * (size_t)n);
   const size_t o_alpha = na_take(off, 8 * (size_t)n);
   const size_t o_G = na_take(off, 8 * (size_t)nsteps * (size_t)g_batch);
+  if (off > cap && waves)
+    return noalloc_pass(ctx, p, batch, Et, alpha_w, G, g_batch, beta_op, ApFT, stepMods, status,
+                        false);
   if (off > cap)
     return fail(ctx, OFX_E_ARG,
                 "N=%d, NSteps=%d, batch=%d needs %zu bytes of device scratch; the no-allocation "
@@ -1622,4 +1616,23 @@ extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params*
     if (na_status[b] == ST_NONFINITE)
       return fail(ctx, OFX_E_NONFINITE, "instance %d: field became non-finite", b);
   return OFX_OK;
+}
+
+extern "C" int ofx_crystal_pass_noalloc(ofx_context* ctx, const ofx_pass_params* p, int batch,
+                                        float* Et, const float* alpha_w, const float* G,
+                                        int g_batch, const float* beta_op, float* ApFT,
+                                        float* stepMods, int* status) {
+  if (!ctx) return OFX_E_ARG;
+  int st = check_pass(ctx, p);
+  if (st) return st;
+  if (batch == 0) return OFX_OK;
+  if (batch < 0 || !Et || !alpha_w || !G || !beta_op)
+    return fail(ctx, OFX_E_ARG, "Et, alpha_w, G, beta_op are required and batch >= 0");
+  if (g_batch != 1 && g_batch != batch)
+    return fail(ctx, OFX_E_ARG, "G must hold NSteps or NSteps*batch values (g_batch=%d)", g_batch);
+  if (batch > NA_MAX_BATCH)
+    return fail(ctx, OFX_E_ARG, "the no-allocation pass takes at most %d instances (got %d)",
+                NA_MAX_BATCH, batch);
+  std::lock_guard<std::mutex> lock(g_na_mu);
+  return noalloc_pass(ctx, p, batch, Et, alpha_w, G, g_batch, beta_op, ApFT, stepMods, status, true);
 }
