@@ -483,9 +483,11 @@ struct WvRun : GEO {
   }
 
   // The own rows of t1 (and, for an attempt of the pass, the cluster's error
-  // records) into the first row pass's elements; *emax = the cluster's error
-  // maximum.  Meets; false (uniform) when the cluster gave up.
-  OFX_DEV bool rows_in(unsigned x, unsigned tag, bool records, double* emax) {
+  // records) into the first row pass's elements.  With records in a cluster of
+  // several workgroups the caller meets before it reads the cluster's error
+  // maximum in red[32] and whether a poll gave up in sflag[1]; otherwise this
+  // meets, and only sflag[1] is set.
+  OFX_DEV void rows_in(unsigned x, unsigned tag, bool records) {
     const int act = row_waves(), l4 = n1 >> 2, qn = 256 >> lg1;
     if (Cn == 1) {
       meet();
@@ -496,7 +498,7 @@ struct WvRun : GEO {
         for (int m = 0; m < 4; m++) t.v[m] = p[wv_pad((t.qr << lg1) + t.jr + l4 * m)];
       });
       wv_order();
-      return true;
+      return;
     }
     const u64* t1 = t1_of(x);
     bool ok = true;
@@ -532,7 +534,6 @@ struct WvRun : GEO {
     }
 #endif
     if (!records) meet();
-    return true;
   }
 
   // Own and halo columns of the inverse transform, scaled, into A0.  Meets
@@ -627,7 +628,7 @@ struct WvRun : GEO {
 
   // one adaptive RK23 pass (ofx_wave_rk23.h)
   OFX_DEV int rk23(R cc, long long& att, long long& acc, double& s_held);
-  OFX_DEV bool boundary_in(unsigned x, unsigned tag, C* dst);
+  OFX_DEV void boundary_in(unsigned x, unsigned tag, C* dst);
 
   OFX_DEV void run(int rank_, C* lds);
 };
@@ -792,7 +793,7 @@ OFX_DEV void WvRun<R, S, GEO, REFRESH>::run(int rank_, C* lds) {
         }
       }
       columns_forward([&](int cl, int r) { return X[wv_pad((cl << lg2) + r)]; }, x1, tag1);
-      rows_in(x1, tag1, true, &gmax);
+      rows_in(x1, tag1, true);
       fft<-1, true>(lg1, row_waves(), Tb);
       if (!early) {
         meet();
@@ -889,7 +890,7 @@ OFX_DEV void WvRun<R, S, GEO, REFRESH>::run(int rank_, C* lds) {
     {
       const unsigned xc1 = ++sy.nx, tagc1 = sy.base + xc1;
       columns_forward([&](int cl, int r) { return A0[(HW + cl) * sT + r]; }, xc1, tagc1);
-      rows_in(xc1, tagc1, false, nullptr);
+      rows_in(xc1, tagc1, false);
       if (sflag[1]) {
         status = ST_BARRIER_TIMEOUT;
         break;

@@ -20,9 +20,10 @@
 namespace ofx {
 
 // The neighbours' K4 boundary columns of exchange x (kx, see rk23_pass) into
-// the halo columns 1..3 and HW + W.. of dst; false in a thread that gave up.
+// the halo columns 1..3 and HW + W.. of dst.  The caller meets before it reads dst
+// or sflag[1], which a poll that gave up sets.
 template <typename R, int S, typename GEO, bool REFRESH>
-OFX_DEV bool WvRun<R, S, GEO, REFRESH>::boundary_in(unsigned x, unsigned tag, C* dst) {
+OFX_DEV void WvRun<R, S, GEO, REFRESH>::boundary_in(unsigned x, unsigned tag, C* dst) {
   const int act = row_waves(), w0 = act < nw ? act : 0, stride = (nw - w0) * 64;
   const u64* kx = (const u64*)uniform(cd.kx) + (size_t)(x & 1u) * Cn * 6 * n2 * TT::NW;
   const int left = (rank + Cn - 1) & (Cn - 1), right = (rank + 1) & (Cn - 1);
@@ -52,7 +53,6 @@ OFX_DEV bool WvRun<R, S, GEO, REFRESH>::boundary_in(unsigned x, unsigned tag, C*
     }
     if (!ok) sflag[1] = 1;
   });
-  return ok;
 }
 
 template <typename R, int S, typename GEO, bool REFRESH>
@@ -219,7 +219,7 @@ OFX_DEV int WvRun<R, S, GEO, REFRESH>::rk23(R cc, long long& att, long long& acc
       }
     }
     columns_forward([&](int cl, int r) { return X[wv_pad((cl << lg2) + r)]; }, x1, tag1);
-    rows_in(x1, tag1, true, &gmax);
+    rows_in(x1, tag1, true);
     if (!early) boundary_in(x1, tag1, Kn);
     fft<-1, true>(lg1, row_waves(), Tb);
     if (!early) {
