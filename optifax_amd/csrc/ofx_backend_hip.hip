@@ -175,8 +175,9 @@ int be_create(int device, Backend** out, DeviceInfo* info) {
     for (int prec : {OFX_F32, OFX_F64})
       for (int lg = WAVE_FIXED_LG; lg <= 16; lg++)
         for (int rk23 : {0, (int)XMODE_RK23_LDS})
-          ok = ok && hipFuncSetAttribute(pass_fn(prec, lg << XMODE_FIXED_SHIFT | rk23),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, dyn) == hipSuccess;
+          if (const void* fn = pass_fn(prec, lg << XMODE_FIXED_SHIFT | rk23))
+            ok = ok && hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, dyn) ==
+                           hipSuccess;
     if (!ok)
       snprintf(info->name + strlen(info->name), sizeof info->name - strlen(info->name),
                " [dyn-LDS attribute not set]");

@@ -45,7 +45,10 @@ __global__ void __launch_bounds__((FixedGeometry<R, LG>::g.block)) wave_rk23_fix
   __shared__ int sflag[4];
   typedef FixedGeometry<R, LG> F;
   // (512 threads form their addresses again each step: kept they spill, 2^15
-  // points 12.1 against 9.3 us per step)
+  // points 12.1 against 9.3 us per step, and still use 152 to 356 bytes of scratch
+  // a lane.  FP64 keeps them, with 68 to 536 bytes of scratch from 2^10 on; kept /
+  // formed again: 2^8 4.0 / 4.2, 2^10 7.7 / 7.4, 2^11 9.0 / 8.6, 2^12 8.9 / 9.9, 2^13
+  // 11.5 / 12.5, 2^14 17.4 / 16.2, 2^15 15.4 / 13.8)
   WvThread<R, F::S, 4> thr;
   wave_main<R, F::S, typename F::Geo, (F::g.block > 256)>(a, (int)blockIdx.x,
                                              reinterpret_cast<cpx<R>*>(ofx_lds_raw), red, sflag,
@@ -63,7 +66,9 @@ static const void* by_size(int lg) {
     case 13: return (const void*)wave_rk23_fixed<R, 13>;
     case 14: return (const void*)wave_rk23_fixed<R, 14>;
     case 15: return (const void*)wave_rk23_fixed<R, 15>;
-    default: return (const void*)wave_rk23_fixed<R, 16>;
+    default:   // (FP64 fields of 2^16 points do not fit LDS on 64 workgroups)
+      if constexpr (sizeof(R) == 4) return (const void*)wave_rk23_fixed<R, 16>;
+      return nullptr;
   }
 }
 
