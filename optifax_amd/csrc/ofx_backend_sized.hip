@@ -6,7 +6,10 @@
 // full) and is bound by instruction issue with two waves a SIMD (LDS holds one
 // workgroup a CU).  32 cavities of 2^14 to 2^16 points, one round trip: 87.8 ms
 // with the geometry read at run time, 82.7 fixed, 76.9 with the stages in one
-// pass.  1024 threads have 128 registers each and spill: 83.2 (against 82.7).
+// pass.  1024 threads have 128 registers each and spill more: 83.2 (against 82.7).
+// The six inlined bodies share one allocation of 256 registers and spill: FP32 103
+// vector and 689 scalar registers (400 bytes of scratch a lane), FP64 324 and 1153
+// (604 bytes); how much time that takes has not been measured.
 #define OFX_NT 512
 #define OFX_SIZED
 #include <hip/hip_runtime.h>

@@ -9,9 +9,11 @@
 
 namespace ofx {
 
-// MAXT: workgroups of up to 256 threads have 512 registers a lane, enough to
-// hold a lane's twiddles, factors and phasors without scratch memory; with
-// 512 threads half of that, and part of them spills.
+// MAXT: workgroups of up to 256 threads have 512 registers a lane (half of them
+// accumulation registers), which hold a lane's twiddles, factors and phasors
+// without scratch memory, in FP64 with the addresses formed again each step.  With
+// 512 threads 256, and part of them spills: FP32 132 to 168 bytes of scratch a
+// lane, FP64 888 to 968 (by default only FP32 fields have 512 threads).
 template <typename R, int S, int MAXT>
 __global__ void __launch_bounds__(MAXT) wave_kernel(LaunchArgs a) {
   extern __shared__ __align__(16) unsigned char ofx_lds_raw[];

@@ -1,5 +1,7 @@
 // The wave kernels (ofx_wave_impl.h) with a grid size's default geometry fixed
 // at compile time (wave_geometry), 2^8 to 2^16 points in either precision.
+// Scratch bytes a lane (addresses kept, see refresh()): FP32 2^10 16, 2^16 368; FP64
+// 2^11 156, 2^13 256, 2^14 140, 2^15 296, 2^16 68; none at the other sizes.
 #include <hip/hip_runtime.h>
 
 #include "../../include/optifax_hip.h"

@@ -31,9 +31,13 @@ namespace ofx {
 
 // Where this kernel runs: FP64 fields from 2^11 points (at 2^10 it measured
 // 0.97-1.04 of the general kernel's speed) and FP32 fields at 2^13.  On shorter
-// FP32 grids it is faster too (2^12: 1.6 times), but its passes round in
-// another order, and what soliton fission makes of that on the coarser grids
-// (2^11, 2 cm: 6e-5 of the field) is more than a change of kernel may move.
+// FP32 grids it is faster too (2^12: 1.6 times) and as accurate, but its passes
+// round in another order, and soliton fission makes more of that on the coarser
+// grids than a change of kernel is meant to move.  Error against FP64, general /
+// this kernel, and their difference (2 cm, Raman and shock, 5, 7.5 and 10 kW, rtol
+// 1e-6): 2^11 1.2e-5 / 9.6e-6, 1.5e-4 / 1.1e-4, 5.4e-4 / 4.3e-4 and 3.1e-6, 4.6e-5,
+// 2.4e-4; 2^12 2.7e-6 / 3.7e-6, 8.2e-6 / 1.2e-5, 3.9e-5 / 1.3e-5 and 3.1e-6, 1.8e-5,
+// 4.7e-5.
 OFX_HD constexpr bool gw_runs(int lg, bool f64) { return f64 ? lg == 11 || lg == 12 : lg == 13; }
 
 // LDS index of element i: one unused element after each 16
@@ -67,7 +71,8 @@ std::vector<cpx<R>> gw_twiddles(int lg) {
 }
 
 // Ends a group of 4 points of an unrolled loop for the scheduler: with all the
-// points' temporaries in flight at once the kernel spills
+// points' temporaries in flight at once the kernel spills more (as it is FP32 2^13
+// keeps 320 and FP64 2^12 316 bytes of scratch a lane, FP64 2^11 none)
 OFX_DEV void gw_group(int i) {
 #ifndef OFX_EMU
   if ((i & 3) == 3) __builtin_amdgcn_sched_barrier(0);
@@ -165,7 +170,7 @@ struct GwRun {
   int tid;         // the thread's index, its origin hidden (refresh)
 
   // Hides where the index comes from, so that addresses are formed where they
-  // are used instead of being kept in registers throughout (kept, they spill)
+  // are used instead of being kept in registers throughout (kept, more spills)
   OFX_DEV void refresh() {
 #ifndef OFX_EMU
     asm volatile("" : "+v"(tid));

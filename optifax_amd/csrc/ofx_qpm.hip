@@ -232,8 +232,13 @@ extern "C" int ofx_qpm_zsum(int device, int n_out, const double* dk, int n_run, 
   hipEventCreate(&e0);
   hipEventCreate(&e1);
   hipEventRecord(e0, 0);
-  // shares per output: as many as give the device's 1024 SIMDs about 8 waves
-  // each (30000 outputs x 602 runs: 0.080 ms with 16 shares, 0.26 before)
+  // Shares per output: 16 while that is at most 8 waves on each of the device's
+  // 1024 SIMDs, 4 up to 32 waves, then 1 (8 and more).  Device us of 802 runs on
+  // either side of the lines: 2^15 - 1 outputs 66 (16 shares), 2^15 74 (4); 2^19 - 1
+  // 890 (4), 2^19 917 (1).  The first line could lie higher (45000 outputs 99 with 4
+  // shares, 91 at the rate of 16).  Maps of few runs gain nothing from shares: 2^19
+  // outputs x 1 run 17 with 4 shares, 10 with 1, of a 1 ms call.  30000 outputs x 602
+  // runs: 80 with 16 shares, 260 before.
   (n_out < (1 << 15)   ? launch_zsum<16>
    : n_out < (1 << 19) ? launch_zsum<4>
                        : launch_zsum<1>)(n_out, (const double*)b_dk.p, n_run,

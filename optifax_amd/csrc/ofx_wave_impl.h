@@ -24,9 +24,14 @@
 // A step of the multi-wave form has 4 workgroup barriers, of the single-wave
 // form none.
 //
-// Bound: the latency of the step's dependent chain (two exchanges of ~1 us
-// each way plus about 20 LDS round trips, and 5 to 8 cycles for each
-// instruction of a wave that is alone on its SIMD), not arithmetic or memory.
+// Bound: the latency of the step's dependent chain, not arithmetic or memory: two
+// exchanges (one tagged word takes about 0.5 us from one XCD to another), about 20
+// LDS round trips, and 5 to 8 cycles for each instruction of a wave that is alone on
+// its SIMD.  At 2^15 points the waves wait in 69 % of their cycles and issue
+// vector instructions in 18 %.  A step of the same share without exchange (2^8
+// points) takes 2.6 us of the 8.0; how much of the rest the polls of whole
+// columns, the threefold inverse columns (2 own, 4 halo) and the members' spread
+// take has not been measured apart.
 // With the geometry a compile-time constant (WvGeoCt) index arithmetic, address
 // registers and the branches on it go.  One instance, us per adaptive step,
 // FP32, against the general kernel at its best geometry: 2^9 points 3.4 (7.9),
@@ -263,7 +268,12 @@ struct WvRun : GEO {
   // registers across it.  Kept they are 10 % faster with a fixed geometry (2^15
   // points 8.0 against 8.6 us per step) and, where they fit, with a run-time one
   // (FP32 fields in workgroups of 256: 9.0 against 10.0); elsewhere they spill
-  // (FP64 14.6 against 13.4, 512 threads 18.9 against 11.9).
+  // (FP64 14.6 against 13.4, 512 threads 18.9 against 11.9).  The fixed geometries
+  // in FP64 and FP32 2^10 and 2^16 keep them too, though from FP64 2^11 on (but
+  // 2^12) and at FP32 2^16 they use 68 to 368 bytes of scratch a lane for it.
+  // us per step, kept / formed again: FP64 2^8 3.15 / 3.44, 2^10 6.1 / 6.3, 2^11 7.4
+  // / 7.1, 2^12 7.9 / 8.5, 2^13 10.6 / 10.6, 2^14 10.5 / 10.0, 2^15 11.2 / 11.4, 2^16
+  // 16.4 / 15.8; FP32 2^10 4.3 / 5.0, 2^16 10.7 / 10.2.
   OFX_DEV void refresh() {
 #ifndef OFX_EMU
     if constexpr (REFRESH)
