@@ -398,8 +398,9 @@ int exchange_mode(int exchange, int cmin) {
 // 2^13 30.6 / 27.3, 2^15 33.0 / 30.7 (its fixed splits are newer than the fit).  That
 // it leans to the wave kernel is wanted: a cluster's last instances run on a device
 // that is no longer full, where that kernel gains most.  With both fitted within
-// 10 %, 300 FP32 cavities of 2^11 took 41.1 us a step in place of 33.9, and five FP64
-// ones of 2^15 and 2^16 5.1 ms in place of 3.8.
+// 10 %, 300 FP32 cavities of 2^11 took 41.9 us a step in place of 33.8; with the wave
+// kernel's 2^16 alone raised by 1.3, five FP64 ones of 2^15 and 2^16 took 5.1 ms in
+// place of 3.8.
 double step_us(const ofx_pass_params& p, int C, bool f64, bool wave) {
   const double x = ilog2i(p.n) - 14, share = (double)p.n / C;
   const bool rk23 = p.method == OFX_METHOD_RK23;
